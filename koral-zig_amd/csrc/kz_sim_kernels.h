@@ -82,8 +82,9 @@ __device__ __forceinline__ void wavespeeds_pass(const GridD &g, const Dev &d, co
   tsd /= ph.tsteplim;
   d.scal[SC_TSTEPDEN * n + c] = tsd;
   if (tsd == tsd) {
-    atomicMax((long long *)&d.tsd[0], dbits(tsd));
-    atomicMin((long long *)&d.tsd[1], dbits(tsd));
+    long long *b = (long long *)slot_of(d.tsd);
+    atomicMax(&b[0], dbits(tsd));
+    atomicMin(&b[1], dbits(tsd));
   }
 }
 
@@ -126,7 +127,7 @@ __device__ __forceinline__ void u2p_pass(const GridD &g, const Dev &d, const kz_
       int fh = ret < -1 ? 1 : 0, fr = corr ? -1 : 0;
       d.flags[KZ_FLAG_HD_FIXUP * n + c] = fh;
       d.flags[KZ_FLAG_RAD_FIXUP * n + c] = fr;
-      if (guard) atomicAdd(&d.cnt[3], (unsigned long long)guard);
+      if (guard) atomicAdd(&slot_of(d.cnt)[3], (unsigned long long)guard);
       if ((fix_hd && fh) || (fix_rad && fr)) {
         unsigned k = atomicAdd(&d.sync[SY_NFIX], 1u);
         d.fix_list[k] = (int32_t)t;
@@ -333,7 +334,7 @@ __device__ __forceinline__ void face_tile(const GridD &g, const Dev &d, const kz
     ag = kzm_fmax(d.scal[(SC_AHD + dim) * n + cf], d.scal[(SC_AHD + dim) * n + cm]);
     agr = kzm_fmax(d.scal[(SC_ARAD + dim) * n + cf], d.scal[(SC_ARAD + dim) * n + cm]);
     fi = fidx(g, dim, cell[0], cell[1], cell[2]);
-    if (guard) atomicAdd(&d.cnt[3], (unsigned long long)guard);
+    if (guard) atomicAdd(&slot_of(d.cnt)[3], (unsigned long long)guard);
   }
   // phase 3: the two sides of a face are neighbouring lanes; each takes the
   // other's flux and conserved vector and writes the LAXF flux of half the
@@ -399,7 +400,7 @@ struct ImpWork {
   int32_t *slow;                  // cells that need rungs past the first
   int32_t *list;                  // [2][n] cells by starting block (MHD, RAD)
   unsigned long long *nslow;      // length of `slow`
-  unsigned long long *ncnt;       // [2] lengths of the two lists
+  unsigned long long *ncnt;       // lengths of the two lists: MHD in the low 32 bits, RAD in the high ones
   // batches (null for grids): the cells the persistent first rung left,
   // rl = [2][n] by starting block (MHD, RAD) with lengths rc = [2], and the
   // queue claim positions qpos (first rung RAD, MHD; the later-rung ladder)
@@ -442,14 +443,15 @@ struct GridCells {
     st(d.u, g.ncell, c, uu);
     st(d.p, g.ncell, c, ppw);
     d.flags[KZ_FLAG_RADIMP_FIXUP * g.ncell + c] = 0;
-    atomicAdd(&d.cnt[1], (unsigned long long)iters);
-    atomicAdd(&d.cnt[2], 1ULL);
+    unsigned long long *k = slot_of(d.cnt);
+    atomicAdd(&k[1], (unsigned long long)iters);
+    atomicAdd(&k[2], 1ULL);
   }
   __device__ void failed(long t) const {
     long ix, iy, iz;
     ijk(t, ix, iy, iz);
     d.flags[KZ_FLAG_RADIMP_FIXUP * g.ncell + cidx(g, ix, iy, iz)] = -1;
-    atomicAdd(&d.cnt[0], 1ULL);
+    atomicAdd(&slot_of(d.cnt)[0], 1ULL);
   }
 };
 // n independent cells (solveImplicitLab per record, implicit.zig:927-1009):
@@ -460,7 +462,7 @@ struct BatchCells {
   const double *dtv;  // [n]
   double *uu, *pp;    // [NV][n]
   kz_implicit_result *res;
-  unsigned long long *cnt;  // [0] failures [1] iterations [2] solves
+  unsigned long long *cnt;  // [NSLOT][SLOT_W]: [0] failures [1] iterations [2] solves
   __device__ long count() const { return n; }
   __device__ bool skip(const kz_physics &, long) const { return false; }
   __device__ void load_p(long t, double *p) const { ld(pp, n, t, p); }
@@ -473,12 +475,13 @@ struct BatchCells {
     st(uu, n, t, u);
     st(pp, n, t, ppw);
     res[t] = kz_implicit_result{1, ir, iters, wp, we, wf};
-    atomicAdd(&cnt[1], (unsigned long long)iters);
-    atomicAdd(&cnt[2], 1ULL);
+    unsigned long long *k = slot_of(cnt);
+    atomicAdd(&k[1], (unsigned long long)iters);
+    atomicAdd(&k[2], 1ULL);
   }
   __device__ void failed(long t) const {
     res[t] = kz_implicit_result{0, -1, 0, WP_RAD, WE_ENERGY, WF_LAB};
-    atomicAdd(&cnt[0], 1ULL);
+    atomicAdd(&slot_of(cnt)[0], 1ULL);
   }
 };
 // The cells of several runs as one sequence (a run group's implicit pass):
@@ -586,14 +589,16 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_PREP) k_imp_prep(S s, ImpWor
     st_tgas = st00.tgas;
   }
   // gather the cell into the list of its starting block, so that each
-  // first-rung kernel runs full waves of one Newton variant
-  if (sw == WP_MHD) {
-    unsigned long long k = atomicAdd(&w.ncnt[0], 1ULL);
-    w.list[k] = (int32_t)t;
-  } else {
-    unsigned long long k = atomicAdd(&w.ncnt[1], 1ULL);
-    w.list[nd + k] = (int32_t)t;
-  }
+  // first-rung kernel runs full waves of one Newton variant: the wave (a
+  // block) asks for its places in both lists with one atomic, whose answer is
+  // not looked at before the bisection is done, so that the wave does not
+  // stand in the queue of one address (12 ns per atomic, 2160 waves at
+  // 384x360, two lists before)
+  const unsigned long long m_mhd = __ballot(sw == WP_MHD), m_rad = __ballot(sw != WP_MHD);
+  const int leader = __ffsll(m_mhd | m_rad) - 1;
+  unsigned long long base = 0;
+  if ((int)threadIdx.x == leader)
+    base = atomicAdd(w.ncnt, ((unsigned long long)__popcll(m_rad) << 32) | (unsigned long long)__popcll(m_mhd));
   ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
   if (ph.implicit.start_with_bisect) {
     solve_1d_prim(pp00, st_ehat, st_ut, st_tgas, dt, cx, pp0);
@@ -602,7 +607,14 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_PREP) k_imp_prep(S s, ImpWor
     for (int i = 0; i < NV; ++i) pp0[i] = pp00[i];
   }
   st(w.pp0, nd, t, pp0);
+  base = __shfl(base, leader);
+  const unsigned long long below = (1ULL << threadIdx.x) - 1ULL;
+  if (sw == WP_MHD) w.list[(long)(base & 0xffffffffULL) + __popcll(m_mhd & below)] = (int32_t)t;
+  else w.list[nd + (long)(base >> 32) + __popcll(m_rad & below)] = (int32_t)t;
 }
+// lengths of the starting-block lists that k_imp_prep filled
+__device__ __forceinline__ long n_mhd(const ImpWork &w) { return (long)(*w.ncnt & 0xffffffffULL); }
+__device__ __forceinline__ long n_rad(const ImpWork &w) { return (long)(*w.ncnt >> 32); }
 __device__ __forceinline__ void imp_load(const ImpWork &w, long nd, long t, double *uu00, double *pp0, State0 &s0,
                                          LagOpac &lag) {
   ld(w.uu00, nd, t, uu00);
@@ -619,7 +631,7 @@ __device__ __forceinline__ void imp_load(const ImpWork &w, long nd, long t, doub
 template <class S, int WP>
 __device__ __forceinline__ void rung0_cell(const S &s, const ImpWork &w, const kz_physics &ph, long i) {
   constexpr int which = WP == WP_MHD ? 0 : 1;
-  if (i >= (long)w.ncnt[which]) return;
+  if (i >= (WP == WP_MHD ? n_mhd(w) : n_rad(w))) return;
   const long nd = s.count();
   long t = w.list[which * nd + i];
   double uu00[NV], pp0[NV], ppw[NV];
@@ -645,7 +657,7 @@ __device__ __forceinline__ void rung0_cell(const S &s, const ImpWork &w, const k
 template <class S, bool BR>
 __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_rung0(S s, ImpWork w, kz_physics ph) {
   ph.opac.synchrotron_bridge = BR;
-  const long brad = ((long)w.ncnt[1] + 63) / 64;
+  const long brad = (n_rad(w) + 63) / 64;
   const long b = blockIdx.x;
   if (b < brad) rung0_cell<S, WP_RAD>(s, w, ph, b * 64 + threadIdx.x);
   else rung0_cell<S, WP_MHD>(s, w, ph, (b - brad) * 64 + threadIdx.x);
@@ -731,9 +743,9 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_rung0_persist(S
   ph.opac.synchrotron_bridge = BR;
   const long nd = s.count();
   const RungDone<S> dr{&s, &w, &ph, 0, 1, WP_RAD, WE_ENERGY, WF_LAB};
-  drain_queue<S, WP_RAD>(s, w, ph, w.list + nd, (long)w.ncnt[1], &w.qpos[0], WE_ENERGY, WF_LAB, dr);
+  drain_queue<S, WP_RAD>(s, w, ph, w.list + nd, n_rad(w), &w.qpos[0], WE_ENERGY, WF_LAB, dr);
   const RungDone<S> dm{&s, &w, &ph, 0, 0, WP_MHD, WE_ENERGY, WF_LAB};
-  drain_queue<S, WP_MHD>(s, w, ph, w.list, (long)w.ncnt[0], &w.qpos[1], WE_ENERGY, WF_LAB, dm);
+  drain_queue<S, WP_MHD>(s, w, ph, w.list, n_mhd(w), &w.qpos[1], WE_ENERGY, WF_LAB, dm);
 }
 // Rungs 1..5 of level 0 (implicit.zig:961-968) over the cells the first
 // rung left (both starting-block lists, MHD start then RAD start), work
@@ -823,7 +835,7 @@ __global__ void __launch_bounds__(64) k_imp_slow(S s, ImpWork w, kz_physics ph, 
   ph.opac.synchrotron_bridge = BR;
   long i = TID;
   // the first-rung lists have been consumed; clear them for the next pass
-  if (i == 0) w.ncnt[0] = w.ncnt[1] = 0;
+  if (i == 0) *w.ncnt = 0;
   if (i >= (long)*w.nslow) return;
   const long nd = s.count();
   long t = w.slow[i];

@@ -1143,9 +1143,22 @@ __device__ __forceinline__ bool dom_cell(const GridD &g, long t, long &c) {
 // coefficients, the CFL accumulators reset; ut0 = u.
 __global__ void k_begin_step(GridD g, Dev d, double forced, int use_forced) {
   long t = TID, c;
+  long long tmaxb = 0;
+  if (t < 64) {  // the first wave folds the slots of the CFL maximum and clears them
+    static_assert(NSLOT == 64, "one slot per lane");
+    long long *b = (long long *)d.tsd + t * SLOT_W;
+    tmaxb = b[0];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const long long v = __shfl_xor(tmaxb, o);
+      tmaxb = v > tmaxb ? v : tmaxb;
+    }
+    b[0] = __double_as_longlong(-1.0);
+    b[1] = __double_as_longlong(1.0e50);
+  }
   if (t == 0) {
     double *ss = d.ss;
-    double tmax = __longlong_as_double((long long)d.tsd[0]);
+    double tmax = __longlong_as_double(tmaxb);
     double own = 1.0 / tmax;
     double dt = use_forced ? forced : own;
     const double gm = GAM_IMEX;
@@ -1158,8 +1171,6 @@ __global__ void k_begin_step(GridD g, Dev d, double forced, int use_forced) {
     ss[SS_NINV_DT] = -1.0 / dt;
     ss[SS_C12] = dt * (1.0 - 2.0 * gm);
     ss[SS_HALF] = dt / 2.0;
-    d.tsd[0] = (unsigned long long)__double_as_longlong(-1.0);
-    d.tsd[1] = (unsigned long long)__double_as_longlong(1.0e50);
   }
   if (!dom_cell(g, t, c)) return;
   long n = g.ncell;
@@ -1278,8 +1289,8 @@ __global__ void k_init_tsd(GridD g, Dev d, double tsd) {
   long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
   d.scal[SC_TSTEPDEN * g.ncell + cidx(g, ix, iy, iz)] = tsd;
   if (t == 0) {
-    d.tsd[0] = (unsigned long long)__double_as_longlong(tsd);
-    d.tsd[1] = (unsigned long long)__double_as_longlong(tsd);
+    for (int k = 0; k < NSLOT; ++k)
+      d.tsd[k * SLOT_W] = d.tsd[k * SLOT_W + 1] = (unsigned long long)__double_as_longlong(tsd);
   }
 }
 
@@ -1385,6 +1396,17 @@ static int dalloc(kz_sim *s, void **p, size_t bytes) {
   s->allocs.push_back(*p);
   s->dev_bytes += bytes;
   return hipMemsetAsync(*p, 0, bytes, s->stream) == hipSuccess ? 0 : KZ_E_HIP;  // ordered before any use
+}
+// every slot of the CFL bounds
+static int put_tsd(kz_sim *s, double tmax, double tmin) {
+  unsigned long long b[NSLOT * SLOT_W] = {};
+  for (int k = 0; k < NSLOT; ++k) {
+    b[k * SLOT_W] = (unsigned long long)__builtin_bit_cast(long long, tmax);
+    b[k * SLOT_W + 1] = (unsigned long long)__builtin_bit_cast(long long, tmin);
+  }
+  HIPCHK(hipMemcpyAsync(s->d.tsd, b, sizeof b, hipMemcpyHostToDevice, s->stream));
+  HIPCHK(hipStreamSynchronize(s->stream));
+  return 0;
 }
 
 
@@ -1492,8 +1514,8 @@ kz_sim *kz_sim_create(const kz_grid *gr, const kz_physics *ph, const double *g, 
   first_err(e, dalloc(s, (void **)&D.kris, (size_t)G.ncell * KR_NC * sizeof(double)));
   size_t nbcx = (size_t)gr->nz * gr->ny * gr->ng * BCX_REC;
   first_err(e, dalloc(s, (void **)&D.bcx, nbcx * sizeof(double)));
-  first_err(e, dalloc(s, (void **)&D.cnt, 8 * sizeof(unsigned long long)));
-  first_err(e, dalloc(s, (void **)&D.tsd, 2 * sizeof(unsigned long long)));
+  first_err(e, dalloc(s, (void **)&D.cnt, (NSLOT * SLOT_W + 1) * sizeof(unsigned long long)));
+  first_err(e, dalloc(s, (void **)&D.tsd, NSLOT * SLOT_W * sizeof(unsigned long long)));
   first_err(e, dalloc(s, (void **)&D.err, sizeof(int)));
   first_err(e, dalloc(s, (void **)&D.ss, SS_N * sizeof(double)));
   long nd = (long)gr->nx * gr->ny * gr->nz;
@@ -1503,7 +1525,7 @@ kz_sim *kz_sim_create(const kz_grid *gr, const kz_physics *ph, const double *g, 
   first_err(e, dalloc(s, (void **)&D.imp_slow, (size_t)nd * sizeof(int32_t)));
   first_err(e, dalloc(s, (void **)&D.imp_nslow, sizeof(unsigned long long)));
   first_err(e, dalloc(s, (void **)&D.imp_list, (size_t)2 * nd * sizeof(int32_t)));
-  first_err(e, dalloc(s, (void **)&D.imp_ncnt, 2 * sizeof(unsigned long long)));
+  first_err(e, dalloc(s, (void **)&D.imp_ncnt, sizeof(unsigned long long)));
   first_err(e, dalloc(s, (void **)&D.imp_rl, (size_t)2 * nd * sizeof(int32_t)));
   first_err(e, dalloc(s, (void **)&D.imp_rc, 2 * sizeof(unsigned long long)));
   first_err(e, dalloc(s, (void **)&D.imp_qpos, 3 * sizeof(unsigned long long)));
@@ -1547,10 +1569,7 @@ kz_sim *kz_sim_create(const kz_grid *gr, const kz_physics *ph, const double *g, 
   }
   s->t_host = 0;
   s->nstep = 0;
-  unsigned long long tsd0[2] = {(unsigned long long)__builtin_bit_cast(long long, 0.0),
-                                (unsigned long long)__builtin_bit_cast(long long, 1.0e50)};
-  if (hipMemcpyAsync(D.tsd, tsd0, sizeof tsd0, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
-      hipStreamSynchronize(s->stream) != hipSuccess) {
+  if (put_tsd(s, 0.0, 1.0e50)) {
     *err = KZ_E_HIP;
     kz_sim_destroy(s);
     return nullptr;
@@ -2094,7 +2113,7 @@ int kz_group_set_runs(kz_group *G, kz_sim *const *sims, int nsims) {
     first_err(e, group_alloc(G, (void **)&G->w.slow, (size_t)c * sizeof(int32_t)));
     first_err(e, group_alloc(G, (void **)&G->w.list, (size_t)2 * c * sizeof(int32_t)));
     first_err(e, group_alloc(G, (void **)&G->w.nslow, sizeof(unsigned long long)));
-    first_err(e, group_alloc(G, (void **)&G->w.ncnt, 2 * sizeof(unsigned long long)));
+    first_err(e, group_alloc(G, (void **)&G->w.ncnt, sizeof(unsigned long long)));
     first_err(e, group_alloc(G, (void **)&G->w.rl, (size_t)2 * c * sizeof(int32_t)));
     first_err(e, group_alloc(G, (void **)&G->w.rc, 2 * sizeof(unsigned long long)));
     first_err(e, group_alloc(G, (void **)&G->w.qpos, 3 * sizeof(unsigned long long)));
@@ -2239,7 +2258,7 @@ int kz_group_sync(kz_group *G) {
 }
 
 int kz_sim_postinit(kz_sim *s, double maxbeta, double *fac_out) {
-  unsigned long long *dmax = s->d.cnt + 7;
+  unsigned long long *dmax = s->d.cnt + NSLOT * SLOT_W;
   HIPCHK(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), s->stream));
   k_beta_max<<<nblk(ndom(s), 256), 256, 0, s->stream>>>(s->g, s->d, s->ph, dmax);
   unsigned long long bits = 0;
@@ -2267,21 +2286,23 @@ int kz_sim_set_time(kz_sim *s, double t, double tstepdenmax, double tstepdenmin)
   HIPCHK(hipStreamSynchronize(s->stream));
   double tt = t;
   HIPCHK(hipMemcpyAsync(s->d.ss + SS_T, &tt, sizeof tt, hipMemcpyHostToDevice, s->stream));
-  unsigned long long b[2] = {(unsigned long long)__builtin_bit_cast(long long, tstepdenmax),
-                             (unsigned long long)__builtin_bit_cast(long long, tstepdenmin)};
-  HIPCHK(hipMemcpyAsync(s->d.tsd, b, sizeof b, hipMemcpyHostToDevice, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
-  return 0;
+  return put_tsd(s, tstepdenmax, tstepdenmin);
 }
 
 int kz_sim_counters(kz_sim *s, kz_counters *c) {
   HIPCHK(hipStreamSynchronize(s->stream));
-  unsigned long long cnt[8], tsd[2];
+  unsigned long long cnt[NSLOT * SLOT_W], tsd[NSLOT * SLOT_W];
   double ss[SS_N];
   HIPCHK(hipMemcpyAsync(cnt, s->d.cnt, sizeof cnt, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipMemcpyAsync(tsd, s->d.tsd, sizeof tsd, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipMemcpyAsync(ss, s->d.ss, sizeof ss, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
+  for (int k = 1; k < NSLOT; ++k) {
+    for (int i = 0; i < 4; ++i) cnt[i] += cnt[k * SLOT_W + i];
+    const long long hi = (long long)tsd[k * SLOT_W], lo = (long long)tsd[k * SLOT_W + 1];
+    if (hi > (long long)tsd[0]) tsd[0] = (unsigned long long)hi;
+    if (lo < (long long)tsd[1]) tsd[1] = (unsigned long long)lo;
+  }
   c->t = ss[SS_T];
   c->dt = ss[SS_DT];
   c->own_dt = ss[SS_OWN_DT];
@@ -2636,7 +2657,7 @@ static int balloc(kz_implicit_batch *b, void **p, size_t bytes) {
 __global__ void k_batch_reset(long n, const double *pp_in, double *pp, double *uu, kz_implicit_result *res,
                               unsigned long long *cnt) {
   long t = TID;
-  if (t < 3) cnt[t] = 0;
+  if (t < NSLOT * SLOT_W) cnt[t] = 0;
   if (t >= n) return;
 #pragma unroll
   for (int iv = 0; iv < NV; ++iv) {
@@ -2665,14 +2686,14 @@ kz_implicit_batch *kz_implicit_batch_create(int64_t n, const kz_physics *ph, int
   first_err(e, balloc(b, (void **)&b->dt, (size_t)n * sizeof(double)));
   for (double **f : {&b->uu, &b->pp, &b->pp_in, &b->stage}) first_err(e, balloc(b, (void **)f, (size_t)n * NV * sizeof(double)));
   first_err(e, balloc(b, (void **)&b->res, (size_t)n * sizeof(kz_implicit_result)));
-  first_err(e, balloc(b, (void **)&b->cnt, 4 * sizeof(unsigned long long)));
+  first_err(e, balloc(b, (void **)&b->cnt, NSLOT * SLOT_W * sizeof(unsigned long long)));
   first_err(e, balloc(b, (void **)&b->w.uu00, (size_t)n * NV * sizeof(double)));
   first_err(e, balloc(b, (void **)&b->w.pp0, (size_t)n * NV * sizeof(double)));
   first_err(e, balloc(b, (void **)&b->w.aux, (size_t)n * IMP_NAUX * sizeof(double)));
   first_err(e, balloc(b, (void **)&b->w.slow, (size_t)n * sizeof(int32_t)));
   first_err(e, balloc(b, (void **)&b->w.list, (size_t)2 * n * sizeof(int32_t)));
   first_err(e, balloc(b, (void **)&b->w.nslow, sizeof(unsigned long long)));
-  first_err(e, balloc(b, (void **)&b->w.ncnt, 2 * sizeof(unsigned long long)));
+  first_err(e, balloc(b, (void **)&b->w.ncnt, sizeof(unsigned long long)));
   first_err(e, balloc(b, (void **)&b->w.rl, (size_t)2 * n * sizeof(int32_t)));
   first_err(e, balloc(b, (void **)&b->w.rc, 2 * sizeof(unsigned long long)));
   first_err(e, balloc(b, (void **)&b->w.qpos, 3 * sizeof(unsigned long long)));
@@ -2731,7 +2752,7 @@ int kz_implicit_batch_set(kz_implicit_batch *b, const double *pp, const kz_geom 
 int kz_implicit_batch_solve(kz_implicit_batch *b, double *ms) {
   if (!b->has_input) return KZ_E_INVALID_CONFIG;
   const long n = b->n;
-  k_batch_reset<<<nblk(n < 3 ? 3 : n, 256), 256, 0, b->stream>>>(n, b->pp_in, b->pp, b->uu, b->res, b->cnt);
+  k_batch_reset<<<nblk(n < NSLOT * SLOT_W ? NSLOT * SLOT_W : n, 256), 256, 0, b->stream>>>(n, b->pp_in, b->pp, b->uu, b->res, b->cnt);
   const BatchCells cells{n, b->gp, b->dt, b->uu, b->pp, b->res, b->cnt};
   HIPCHK(hipEventRecord(b->ev[0], b->stream));
   launch_implicit(cells, b->w, b->ph, n, true, b->persist_blocks, b->stream);
@@ -2760,8 +2781,14 @@ int kz_implicit_batch_get(kz_implicit_batch *b, double *uu, double *pp, kz_impli
     HIPCHK(hipStreamSynchronize(b->stream));
   }
   if (r) HIPCHK(hipMemcpyAsync(r, b->res, (size_t)n * sizeof(kz_implicit_result), hipMemcpyDeviceToHost, b->stream));
-  if (counts) HIPCHK(hipMemcpyAsync(counts, b->cnt, 3 * sizeof(uint64_t), hipMemcpyDeviceToHost, b->stream));
+  unsigned long long cnt[NSLOT * SLOT_W];
+  if (counts) HIPCHK(hipMemcpyAsync(cnt, b->cnt, sizeof cnt, hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
+  if (counts)
+    for (int i = 0; i < 3; ++i) {
+      counts[i] = 0;
+      for (int k = 0; k < NSLOT; ++k) counts[i] += cnt[k * SLOT_W + i];
+    }
   return 0;
 }
 
@@ -2776,7 +2803,7 @@ int kz_implicit_batch_get(kz_implicit_batch *b, double *uu, double *pp, kz_impli
 // scalars (IMP_NAUX) as doubles, and five int32 list entries.
 #define NA_DBL_PER_CELL (GEO_NC + 1 + 4 * NV + IMP_NAUX)
 #define NA_INT_PER_CELL 5
-#define NA_NCNT 12  // cnt[4] nslow ncnt[2] rc[2] qpos[3]
+#define NA_NCNT (NSLOT * SLOT_W + 8)  // cnt[NSLOT][SLOT_W] nslow ncnt rc[2] qpos[3], one spare
 static constexpr size_t NA_BYTES =
     ((size_t)KZ_NOALLOC_MAX_CELLS * (NA_DBL_PER_CELL * 8 + NA_INT_PER_CELL * 4) + NA_NCNT * 8 + 255) / 256 * 256;
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
@@ -2810,7 +2837,11 @@ __global__ void k_na_pack(long n, const double *pp_aos, const kz_geom *g, double
 __global__ void k_na_unpack(long n, const double *uu, const double *pp, double *uu_aos, double *pp_aos,
                             const unsigned long long *cnt, uint64_t *counts) {
   long t = TID;
-  if (counts && t < 3) counts[t] = cnt[t];
+  if (counts && t < 3) {
+    uint64_t sum = 0;
+    for (int k = 0; k < NSLOT; ++k) sum += cnt[k * SLOT_W + t];
+    counts[t] = sum;
+  }
   if (t >= n * NV) return;
   long c = t / NV;
   int iv = t % NV;
@@ -2867,10 +2898,10 @@ extern "C" int kz_implicit_solve_noalloc(int64_t n, const double *pp_in, const k
   w.rl = ip + 3 * n;
   unsigned long long *ctr = (unsigned long long *)(((uintptr_t)(ip + 5 * n) + 7) & ~(uintptr_t)7);
   unsigned long long *cnt = ctr;
-  w.nslow = ctr + 4;
-  w.ncnt = ctr + 5;
-  w.rc = ctr + 7;
-  w.qpos = ctr + 9;
+  w.nslow = ctr + NSLOT * SLOT_W;
+  w.ncnt = w.nslow + 1;
+  w.rc = w.nslow + 2;
+  w.qpos = w.nslow + 4;
   kz_physics ph = *phys;
   k_na_pack<<<nblk(n < NA_NCNT ? NA_NCNT : n, 256), 256, 0, st>>>(n, pp_in, g, gp, spp, suu, res, ctr);
   const BatchCells cells{n, gp, dt, suu, spp, res, cnt};
