@@ -26,6 +26,10 @@ HIPCC_FLAGS = [
     # keep hipcc from emitting packed-FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
+    # constants stay where they are used: hoisted out of the solver loops they
+    # need more registers than there are, and each is then read back from a
+    # spill (k_u2p: 256 vector registers and 140 B of scratch against 247)
+    "-mllvm", "-disable-machine-licm",
 ]
 
 

@@ -153,7 +153,7 @@ __global__ void b_u2p_solver_w(long n, const double *uu, double *pp, const kz_ge
     p[k] = pp[i * NV + k];
     u[k] = uu[i * NV + k];
   }
-  ret[i] = u2p_solver_w(u, p, gm, etype, gam);
+  ret[i] = u2p_solver_w(u, p, gm, &etype, false, gam);
   for (int k = 0; k < NV; ++k) pp[i * NV + k] = p[k];
 }
 
@@ -235,11 +235,11 @@ __global__ void b_math(long n, int fn, const double *x, const double *y, double 
   if (i >= n) return;
   double a = x[i], b = y ? y[i] : 0.0, r;
   switch (fn) {
-    case 0: r = kzm_exp(a); break;
-    case 1: r = kzm_log(a); break;
+    case 0: r = dm_exp(a); break;
+    case 1: r = dm_log(a); break;
     case 2: r = kzm_pow(a, b); break;
-    case 3: r = kzm_cbrt(a); break;
-    case 4: r = kzm_log1p(a); break;
+    case 3: r = dm_cbrt(a); break;
+    case 4: r = dm_log1p(a); break;
     case 5: r = kzm_sqrt(a); break;
     default: r = a / b; break;
   }

@@ -16,6 +16,7 @@
 
 #define KZM_QUAL __host__ __device__ static inline
 #include "kz_math.h"
+#include "kz_dev_math.h"
 
 #define KZD __device__ static inline
 
@@ -106,7 +107,7 @@ KZD double alpha_gamma(const double u[4], const Geo &gm) {  // :250-260
 #pragma unroll
     for (int j = 1; j < 4; ++j) qsq += u[i] * u[j] * gm.g[i][j];
   double ag2 = (-1.0 / gm.G[0][0]) * (1.0 + qsq);
-  return ag2 < 0 ? 1.0 : kzm_sqrt(ag2);
+  return dm_sel(ag2 < 0, 1.0, kzm_sqrt(ag2));
 }
 KZD void velr_to_vel4(const double u[4], const Geo &gm, double o[4]) {  // :265-273
   double ag = alpha_gamma(u, gm);
@@ -160,7 +161,7 @@ KZD double s_from_u(double rho, double u, double gam) {  // hydro.zig:32-37
   double gammam1 = gam - 1.0;
   double indexn = 1.0 / gammam1;
   double pre = gammam1 * u;
-  return rho * kzm_log(kzm_pow(pre, indexn) / kzm_pow(rho, indexn + 1.0));
+  return rho * dm_log_entropy(pre, rho, indexn);
 }
 
 // ---- p2u.zig ---------------------------------------------------------------
@@ -335,10 +336,19 @@ KZD void rad_wavespeeds(const double *pp, const Geo &gm, const double tau[3], co
 struct Opac {
   double gas_abs, rad_abs, rad_ross;
 };
+// The channels of a run with everything on (the reference's PUFFY options).
+// One test of the parameter block picks ALL, whose code carries no branch:
+// the dozen transcendentals of a state are independent of each other, and in
+// one block the compiler runs them side by side (kz_dev_math.h).
+KZD bool all_channels(const kz_opac_params &c) {
+  return c.kappa_mode == 0 && c.kappaes_mode == 1 && c.bremsstrahlung && c.synchrotron && c.kleinnishina &&
+         c.comptonization;
+}
 // opacities.zig:131-315 at the .residual / .chi levels (the channels the
 // step consumes); `want_rad` false is the .chi level.
-KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double trad, double ne, double bsq,
-                        bool want_rad) {
+template <bool ALL>
+KZDM Opac calc_opacities(const kz_opac_params &c, double rho, double te, double trad, double ne, double bsq,
+                         bool want_rad) {
   double rt_te = kzm_sqrt(te);
   double rhocgs = c.rhogu2cgs * rho;
   double nethcgs = ne * c.numdensgu2cgs;
@@ -346,7 +356,7 @@ KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double t
   double bmagcgs = kzm_sqrt(bsqcgs);
   double bbenergy = (4.0 * c.sigma_rad_cgs) * te * te * te * te;
   double kgff = 0, krff = 0, krffross = 0, kgsyn = 0, krsyn = 0, krsynross = 0;
-  if (c.bremsstrahlung) {
+  if (ALL || c.bremsstrahlung) {
     double mfrac = 1.0 - c.hfrac - c.hefrac;
     double emis_ff = 1.4e-27 * nethcgs * ((c.hfrac + c.hefrac + c.z2diva_mean * mfrac) / c.m_proton_cgs) * rt_te *
                      1.2 * (1.0 + 4.4e-10 * te);
@@ -355,15 +365,15 @@ KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double t
       double zeta = trad / te;
       double zi = 1.0 / zeta;
       double zi3 = zi * zi * zi;
-      krff = kgff * kzm_log1p(1.6 * zeta) * c.one_over_log_2p6 * zi3;
-      double zr5 = kzm_pow(zeta, 0.2);
+      krff = kgff * dm_log1p(1.6 * zeta) * c.one_over_log_2p6 * zi3;
+      double zr5 = dm_pow_frac(zeta, 0.2);
       double zr5i4 = 1.0 / (zr5 * zr5 * zr5 * zr5);
       double zr5i3 = zr5 * zr5i4;
       double sc = 14.12 / (432.7 - 106.8 * zr5i3 + 43.17 * zr5i4 + 57.88 * zi);
       krffross = kgff * sc * zi3;
     }
   }
-  if (c.synchrotron) {
+  if (ALL || c.synchrotron) {
     // opacities.zig:208-297: with the bridge the synchrotron Trad is clamped
     // up to TradBB^(4/3) / Te^(1/3) (TradBB = trad here: no photon-number
     // evolution), non-relativistic components are added to the gas and
@@ -379,13 +389,13 @@ KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double t
     if (want_rad) {
       double trad_syn = trad;
       if (bridge) {
-        const double trad_lim = kzm_pow(trad, 4.0 / 3.0) / kzm_pow(te, 1.0 / 3.0);
+        const double trad_lim = dm_pow_frac(trad, 4.0 / 3.0) / dm_pow_frac(te, 1.0 / 3.0);
         trad_syn = trad < trad_lim ? trad_lim : trad;
       }
       double nu_mb = 1.19e-13 * te * te;
       double zbr = c.k_boltz_cgs * trad_syn / c.h_cgs / nu_mb;
-      double den = 1.79 * kzm_cbrt(zbr * zbr * zbr * zbr * zbr * bmagcgs * bmagcgs * bmagcgs * bmagcgs) +
-                   1.35 * kzm_cbrt(zbr * zbr * zbr * zbr * zbr * zbr * zbr * bmagcgs * bmagcgs) +
+      double den = 1.79 * dm_cbrt(zbr * zbr * zbr * zbr * zbr * bmagcgs * bmagcgs * bmagcgs * bmagcgs) +
+                   1.35 * dm_cbrt(zbr * zbr * zbr * zbr * zbr * zbr * zbr * bmagcgs * bmagcgs) +
                    0.248 * zbr * zbr * zbr;
       double iab = bmagcgs * bmagcgs / den;
       double te5 = te * te * te * te * te;
@@ -393,28 +403,16 @@ KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double t
       if (bridge)
         krsyn += c.kappacgs2gu *
                  (2.35869e-21 * (nethcgs / rhocgs) * (bmagcgs * bmagcgs) / (trad_syn * trad_syn * trad_syn)) * rho;
-      // two powers of each base: one logarithm per base (kzm_pow_from_log
-      // returns kzm_pow's bits for a finite positive base)
-      double bmb, pb69, pz169, pz463;
-      if (bmagcgs > 0.0 && kzm_isfinite(bmagcgs)) {
-        double lh, ll;
-        kzm_log_dd(bmagcgs, &lh, &ll);
-        bmb = kzm_pow_from_log(lh, ll, -0.463);
-        pb69 = kzm_pow_from_log(lh, ll, 0.69);
-      } else {
-        bmb = bmagcgs > 0.0 ? kzm_pow(bmagcgs, -0.463) : 0.0;
-        pb69 = kzm_pow(bmagcgs, 0.69);
-      }
-      if (zbr > 0.0 && kzm_isfinite(zbr)) {
-        double lh, ll;
-        kzm_log_dd(zbr, &lh, &ll);
-        pz169 = kzm_pow_from_log(lh, ll, 1.69);
-        pz463 = kzm_pow_from_log(lh, ll, 0.463);
-      } else {
-        pz169 = kzm_pow(zbr, 1.69);
-        pz463 = kzm_pow(zbr, 0.463);
-      }
-      double iabr = 0.13 * pb69 / (pz169 * kzm_exp(1.6 * pz463 * bmb));
+      // two powers of each base: one logarithm per base
+      double bh, bl, zh, zl;
+      dm_log_dd(bmagcgs, &bh, &bl);
+      dm_log_dd(zbr, &zh, &zl);
+      const double bmb =
+          dm_sel(bmagcgs > 0.0 && bmagcgs < KZM_INF, dm_pow_from_log(bh, bl, -0.463), 0.0);  // 0 at 0, inf and NaN
+      const double pb69 = dm_pow_fix(bmagcgs, dm_pow_from_log(bh, bl, 0.69));
+      const double pz169 = dm_pow_fix(zbr, dm_pow_from_log(zh, zl, 1.69));
+      const double pz463 = dm_pow_fix(zbr, dm_pow_from_log(zh, zl, 0.463));
+      double iabr = 0.13 * pb69 / (pz169 * dm_exp(1.6 * pz463 * bmb));
       krsynross = c.kappacgs2gu * (2.13e39 * (nethcgs / rhocgs) / te5 * iabr) * rho;
     }
     if (!bridge) {
@@ -433,10 +431,11 @@ KZD Opac calc_opacities(const kz_opac_params &c, double rho, double te, double t
   o.rad_ross = krffross + krsynross;
   return o;
 }
-KZD double kappaes_at(const kz_opac_params &c, double rho, double trad) {  // radforce.zig:140-151
-  if (c.kappaes_mode == 1) {  // opacities.zig:352-360
+template <bool ALL>
+KZDM double kappaes_at(const kz_opac_params &c, double rho, double trad) {  // radforce.zig:140-151
+  if (ALL || c.kappaes_mode == 1) {  // opacities.zig:352-360
     double corr = 1.0;
-    if (c.kleinnishina) corr = 1.0 / (1.0 + kzm_pow(trad / 4.5e8, 0.86));
+    if (ALL || c.kleinnishina) corr = 1.0 / (1.0 + dm_pow_frac(trad / 4.5e8, 0.86));
     return ((0.2 * (1.0 + c.hfrac)) * corr) * c.kappa_cgs2gu_factor * rho;
   }
   if (c.kappaes_mode == 2) return c.kappaes_grey * rho;
@@ -453,8 +452,9 @@ struct RadState {
   Opac op;
 };
 // radforce.zig:241-351 fillRadStateCoreG; `full` computes sgas
-KZD void fill_radstate(const double *pp, const Geo &gm, double gam, const kz_opac_params &c, bool full,
-                       RadState &st) {
+template <bool ALL>
+KZDM void fill_radstate_t(const double *pp, const Geo &gm, double gam, const kz_opac_params &c, bool full,
+                          RadState &st) {
   double rho = pp[RHO], uint = pp[UU];
   double tgas, te;
   temps_from_urho(c, uint, rho, gam, &tgas, &te);
@@ -470,17 +470,23 @@ KZD void fill_radstate(const double *pp, const Geo &gm, double gam, const kz_opa
 #pragma unroll
     for (int j = 0; j < 4; ++j) ehat += st.rij[i][j] * st.ucov[i] * st.ucov[j];
   double trad = lte_t_from_e(c, ehat);
-  st.kappaes = kappaes_at(c, rho, trad);
-  if (c.kappa_mode == 0) {
-    st.op = calc_opacities(c, rho, te, trad, ne, bsq, true);
+  st.kappaes = kappaes_at<ALL>(c, rho, trad);
+  if (ALL || c.kappa_mode == 0) {
+    st.op = calc_opacities<ALL>(c, rho, te, trad, ne, bsq, true);
   } else {
     double kap = c.kappa_grey * rho;
     st.op.gas_abs = kap; st.op.rad_abs = kap; st.op.rad_ross = kap;
   }
   st.tgas = tgas; st.te = te; st.uint = uint; st.ehat = ehat; st.trad = trad;
 }
+KZD void fill_radstate(const double *pp, const Geo &gm, double gam, const kz_opac_params &c, bool full,
+                       RadState &st) {
+  if (all_channels(c)) fill_radstate_t<true>(pp, gm, gam, c, full, st);
+  else fill_radstate_t<false>(pp, gm, gam, c, full, st);
+}
 // radforce.zig:432-494 calcGiFromStateCoreG (slim: ff[0] and lab only)
-KZD void calc_gi(const RadState &st, const kz_opac_params &c, double opdamp, double *giff0, double gilab[4]) {
+template <bool ALL>
+KZDM void calc_gi(const RadState &st, const kz_opac_params &c, double opdamp, double *giff0, double gilab[4]) {
   double b = c.sigma_rad_over_pi * st.te * st.te * st.te * st.te;
   double kra = st.op.rad_abs, kga = st.op.gas_abs, krr = st.op.rad_ross, kes = st.kappaes, ruu = st.ehat;
 #pragma unroll
@@ -491,7 +497,7 @@ KZD void calc_gi(const RadState &st, const kz_opac_params &c, double opdamp, dou
     gilab[i] = -(krr + kes) * ru - ((krr + kes - kra) * ruu + kga * c.fourpi * b) * st.ucon[i];
   }
   double ff0 = -kga * c.fourpi * b + kra * st.ehat;
-  if (c.comptonization) {
+  if (ALL || c.comptonization) {
     double th = c.kb_over_me * st.te;  // radforce.zig:370-375
     double coeff = st.kappaes * st.ehat * ((4.0 * c.kb_over_me) * (st.trad - st.te)) *
                    (1.0 + 3.683 * th + 4.0 * th * th) / (1.0 + 4.0 * th);
@@ -516,8 +522,10 @@ KZD double calc_chi_slim(const double *pp, const Geo &gm, double gam, const kz_o
   ucon_ucov(pp, gm, ucon, ucov);
   double bcon[4], bcov[4], bsq;
   bcon_bcov_bsq(pp[B1], pp[B2], pp[B3], ucon, ucov, gm, bcon, bcov, &bsq);
-  double kappa = c.kappa_mode == 0 ? calc_opacities(c, rho, te, te, ne, bsq, false).gas_abs : c.kappa_grey * rho;
-  return kappa + kappaes_at(c, rho, te);
+  if (all_channels(c)) return calc_opacities<true>(c, rho, te, te, ne, bsq, false).gas_abs + kappaes_at<true>(c, rho, te);
+  double kappa =
+      c.kappa_mode == 0 ? calc_opacities<false>(c, rho, te, te, ne, bsq, false).gas_abs : c.kappa_grey * rho;
+  return kappa + kappaes_at<false>(c, rho, te);
 }
 
 // ---- fv/recon.zig (PPM, :99-195) and laxf.zig ------------------------------

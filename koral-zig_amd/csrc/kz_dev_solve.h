@@ -18,7 +18,7 @@ struct Cons {
   double Qn, Qtsq, D, QdotBsq, Bsq, Sc;
 };
 
-KZD Resid f_u2p(int etype, double Wp, const Cons &c, double pg) {
+KZDM Resid f_u2p(int etype, double Wp, const Cons &c, double pg) {
   double W = Wp + c.D;  // invert.zig:116-210 (both residuals share wKinematics)
   double x = c.Bsq + W;
   double wsq = W * W;
@@ -46,7 +46,7 @@ KZD Resid f_u2p(int etype, double Wp, const Cons &c, double pg) {
   } else {
     double pressure = (pg - 1.0) / pg * wmrho0;
     double indexn = 1.0 / (pg - 1.0);
-    double ss = kzm_log(kzm_pow(pressure, indexn) / kzm_pow(rho0, indexn + 1.0));
+    double ss = dm_log_entropy(pressure, rho0, indexn);
     r.f = -c.Sc + c.D * ss;
     r.err = kzm_fabs(r.f) / (kzm_fabs(c.Sc) + kzm_fabs(c.D * ss));
     double dssdrho = pg / ((1.0 - pg) * rho0);
@@ -61,13 +61,29 @@ KZD Resid f_u2p(int etype, double Wp, const Cons &c, double pg) {
   return r;
 }
 
-KZD bool w_oob(double W, const Cons &c, const Resid &r) {  // invert.zig:221-224
-  return (W * W * W * (W + 2.0 * c.Bsq) - c.QdotBsq * (2.0 * W + c.Bsq)) <= W * W * (c.Qtsq - c.Bsq * c.Bsq) ||
-         !kzm_isfinite(r.f) || !kzm_isfinite(r.df);
+// the two halves of invert.zig:221-224: W below the physical range, and a
+// residual that is no number.  The first needs no residual, so it is asked
+// first.
+KZD bool w_below(double W, const Cons &c) {
+  return (W * W * W * (W + 2.0 * c.Bsq) - c.QdotBsq * (2.0 * W + c.Bsq)) <= W * W * (c.Qtsq - c.Bsq * c.Bsq);
 }
+KZD bool r_bad(const Resid &r) { return !kzm_isfinite(r.f) || !kzm_isfinite(r.df); }
 
-// invert.zig:235-404 u2pSolverW (pp in/out; returns the reference's code)
-KZD int u2p_solver_w(const double *uu, double *pp, const Geo &gm, int etype, double pg) {
+// invert.zig:235-404 u2pSolverW, from the energy equation (etype 0) or the
+// entropy (1), and with `fallback` from the entropy where the energy equation
+// fails (one cell in twenty of a 48x48x16 wedge), which is how its callers use
+// it (invert.zig:441-451, implicit.zig:293-296).  pp in/out; returns the
+// reference's code of the last attempt and in *etype which one that was.
+//
+// The reference evaluates the residual at every trial W and once more, at the
+// same W, where it goes on from it; here the value of an accepted trial is
+// kept for the next iteration (the same arguments, the same bits), so an
+// iteration takes one evaluation instead of two, and a trial below the range
+// (w_below) takes none.  Bracketing, damped trials, the step after a zero
+// derivative and both equations share this one evaluation: a lane that has
+// fallen back runs beside one that has not, and the code stands once.
+KZDM int u2p_solver_w(const double *uu, double *pp, const Geo &gm, int *etype_io, bool fallback, double pg) {
+  int etype = *etype_io;
   double gi = 1.0 / gm.gdet;
   double alpha = gm.alpha;
   Cons c;
@@ -82,126 +98,163 @@ KZD int u2p_solver_w(const double *uu, double *pp, const Geo &gm, int etype, dou
   c.Bsq = dot4(Bcon, Bcov);
   double QdotB = dot4(Qcov, Bcon);
   c.QdotBsq = QdotB * QdotB;
-  double ncov[4] = {-alpha, 0, 0, 0}, ncon[4];
-  raise4(ncov, gm, ncon);
-  c.Qn = Qcon[0] * ncov[0];
+  // n_mu = (-alpha, 0, 0, 0): the reference's full sums over it add only
+  // zeros to these (a metric is finite), and to Qt what 0 * Qcon gives, zero
+  // or NaN
   double Qt[4];
+  {
+    const double zero = 0.0 * Qcon[1] + 0.0 * Qcon[2] + 0.0 * Qcon[3];
+    const double nc = -alpha;
+    c.Qn = Qcon[0] * nc;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    double s = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s += ((i == j ? 1.0 : 0.0) + ncon[i] * ncov[j]) * Qcon[j];
-    Qt[i] = s;
+    for (int i = 0; i < 4; ++i) {
+      const double ncon = 0.0 + nc * gm.G[i][0];
+      const double s = 0.0 + ((i == 0 ? 1.0 : 0.0) + ncon * nc) * Qcon[0];
+      Qt[i] = (i == 0 ? s : s + Qcon[i]) + zero;
+    }
   }
   double Qtcov[4];
   lower4(Qt, gm, Qtcov);
   c.Qtsq = dot4(Qt, Qtcov);
-
-  double qsq = 0;
-#pragma unroll
-  for (int i = 1; i < 4; ++i)
-#pragma unroll
-    for (int j = 1; j < 4; ++j) qsq += pp[VX - 1 + i] * pp[VX - 1 + j] * gm.g[i][j];
-  double W = (pp[RHO] + pg * pp[UU]) * (1.0 + qsq);
   const double conv = 1.0e-10;
 
-  int inc = 0;
+  enum { BRACKET, TRIAL, PLAIN };
+  int mode = BRACKET, tries = 0, iter = 0;
+  double W = 0, Wt = 0, f0 = 0, dfdW = 0, dumpfac = 1.0, errr = 0;
+  bool start = true;
   for (;;) {
-    Resid r = f_u2p(etype, W - c.D, c, pg);
-    if (w_oob(W, c, r) && inc < 50) {
-      W *= 10.0;
-      inc += 1;
-      continue;
-    }
-    break;
-  }
-  if (inc >= 50) return -150;
-  int iter = 0;
-  while (iter < 50) {
-    double Wprev = W;
-    iter += 1;
-    Resid r = f_u2p(etype, W - c.D, c, pg);
-    double f0 = r.f, dfdW = r.df, errr = r.err;
-    if (errr < conv) break;
-    if (dfdW == 0.0) {
-      W *= 1.1;
-      continue;
-    }
-    double Wnew = W - f0 / dfdW;
-    int idump = 0;
-    double dumpfac = 1.0;
-    for (;;) {
-      Resid rt = f_u2p(etype, Wnew - c.D, c, pg);
-      if (w_oob(Wnew, c, rt) && idump < 100) {
-        idump += 1;
-        dumpfac /= 2.0;
-        Wnew = W - dumpfac * f0 / dfdW;
-        continue;
-      }
-      break;
-    }
-    if (idump >= 100) return -101;
-    W = Wnew;
-    if (kzm_fabs(W) > 1.0 / 1.0e-80) return -103;
-    if (kzm_fabs((W - Wprev) / Wprev) < conv && errr < 1.0e-1) break;
-  }
-  if (iter >= 50) return -102;
-  if (!kzm_isfinite(W)) return -103;
-
-  double wsq = W * W;
-  double xsq = (c.Bsq + W) * (c.Bsq + W);
-  double v2 = (wsq * c.Qtsq + c.QdotBsq * (c.Bsq + 2.0 * W)) / (wsq * xsq);
-  double gamma2 = 1.0 / (1.0 - v2);
-  double gamma = kzm_sqrt(gamma2);
-  double rho = c.D / gamma;
-  double entr = c.Sc / gamma;
-  double uint = 1.0 / pg * (W / gamma2 - rho);
-  double ut[4];
+    if (start) {
+      double qsq = 0;
 #pragma unroll
-  for (int i = 1; i < 4; ++i) ut[i] = gamma / (W + c.Bsq) * (Qt[i] + QdotB * Bcon[i] / W);
-  if (!kzm_isfinite(ut[1])) return -120;
-  if (uint < 0.0 || gamma2 < 0.0 || W != W || !kzm_isfinite(W)) return -104;
-  pp[RHO] = rho;
-  pp[UU] = uint;
-  pp[VX] = ut[1];
-  pp[VY] = ut[2];
-  pp[VZ] = ut[3];
-  if (rho < 0.0) return -105;
-  pp[ENTR] = entr;
-  pp[B1] = uu[B1] * gi;
-  pp[B2] = uu[B2] * gi;
-  pp[B3] = uu[B3] * gi;
-  return 0;
+      for (int i = 1; i < 4; ++i)
+#pragma unroll
+        for (int j = 1; j < 4; ++j) qsq += pp[VX - 1 + i] * pp[VX - 1 + j] * gm.g[i][j];
+      Wt = (pp[RHO] + pg * pp[UU]) * (1.0 + qsq);
+      mode = BRACKET;
+      tries = iter = 0;
+      start = false;
+    }
+    Resid r{};
+    bool oob = mode != PLAIN && w_below(Wt, c);
+    if (!oob) {
+      r = f_u2p(etype, Wt - c.D, c, pg);
+      oob = mode != PLAIN && r_bad(r);
+    }
+    int code = 0;
+    bool ends = false;  // this attempt's iteration ends
+    if (oob) {
+      tries += 1;
+      if (mode == BRACKET) {
+        Wt *= 10.0;
+        if (tries >= 50) code = -150;
+      } else {
+        dumpfac /= 2.0;
+        Wt = W - dumpfac * f0 / dfdW;
+        if (tries >= 100) code = -101;
+      }
+    } else {
+      if (mode == TRIAL) {
+        const double Wprev = W;
+        W = Wt;
+        if (kzm_fabs(W) > 1.0 / 1.0e-80) code = -103;
+        else if (kzm_fabs((W - Wprev) / Wprev) < conv && errr < 1.0e-1) ends = true;
+      } else {
+        W = Wt;
+      }
+      if (code == 0 && !ends) {
+        if (iter >= 50) {
+          ends = true;
+        } else {
+          iter += 1;
+          errr = r.err;
+          if (errr < conv) {
+            ends = true;
+          } else if (r.df == 0.0) {
+            Wt = W * 1.1;
+            mode = PLAIN;
+          } else {
+            f0 = r.f;
+            dfdW = r.df;
+            dumpfac = 1.0;
+            tries = 0;
+            mode = TRIAL;
+            Wt = W - f0 / dfdW;
+          }
+        }
+      }
+      if (ends) {
+        if (iter >= 50) code = -102;
+        else if (!kzm_isfinite(W)) code = -103;
+        else {
+          double wsq = W * W;
+          double xsq = (c.Bsq + W) * (c.Bsq + W);
+          double v2 = (wsq * c.Qtsq + c.QdotBsq * (c.Bsq + 2.0 * W)) / (wsq * xsq);
+          double gamma2 = 1.0 / (1.0 - v2);
+          double gamma = kzm_sqrt(gamma2);
+          double rho = c.D / gamma;
+          double entr = c.Sc / gamma;
+          double uint = 1.0 / pg * (W / gamma2 - rho);
+          double ut[4];
+#pragma unroll
+          for (int i = 1; i < 4; ++i) ut[i] = gamma / (W + c.Bsq) * (Qt[i] + QdotB * Bcon[i] / W);
+          if (!kzm_isfinite(ut[1])) code = -120;
+          else if (uint < 0.0 || gamma2 < 0.0 || W != W || !kzm_isfinite(W)) code = -104;
+          else {
+            pp[RHO] = rho;
+            pp[UU] = uint;
+            pp[VX] = ut[1];
+            pp[VY] = ut[2];
+            pp[VZ] = ut[3];
+            if (rho < 0.0) code = -105;
+            else {
+              pp[ENTR] = entr;
+              pp[B1] = uu[B1] * gi;
+              pp[B2] = uu[B2] * gi;
+              pp[B3] = uu[B3] * gi;
+              *etype_io = etype;
+              return 0;
+            }
+          }
+        }
+      }
+    }
+    if (code != 0) {
+      if (etype != 0 || !fallback) {
+        *etype_io = etype;
+        return code;
+      }
+      etype = 1;
+      start = true;
+    }
+  }
 }
 
-// invert.zig:422-467 u2pMhd; returns ret (0/-1/-2/-3), sets *entropy_used
-KZD int u2p_mhd(const double *uu_in, double *pp, const Geo &gm, double gam, const kz_floor_params &f,
-                int *entropy_used) {
-  double uu[NV], pm[NV];
+// invert.zig:422-467 u2pMhd; returns ret (0/-1/-2/-3), sets *entropy_used.
+// A failed solve leaves pp as it came (the reference's ppbak), except that
+// its guess fields are put back here.
+KZDM int u2p_mhd(const double *uu_in, double *pp, const Geo &gm, double gam, const kz_floor_params &f,
+                 int *entropy_used) {
+  double uu[NV];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    uu[i] = uu_in[i];
-    pm[i] = pp[i];
-  }
+  for (int i = 0; i < NV; ++i) uu[i] = uu_in[i];
+  double keep[5] = {pp[RHO], pp[UU], pp[VX], pp[VY], pp[VZ]};
   int ret = 0;
-  *entropy_used = 0;
   if (uu[RHO] * gm.alpha / gm.gdet < 0.0) {
-    pm[RHO] = f.rhofloor;
+    pp[RHO] = f.rhofloor;
     uu[RHO] = f.rhofloor * gm.gdet / gm.alpha;
     ret = -2;
   }
-  int r = u2p_solver_w(uu, pm, gm, 0, gam);
+  int etype = 0;
+  const int r = u2p_solver_w(uu, pp, gm, &etype, true, gam);
+  *entropy_used = etype;
+  if (etype) ret = -1;
   if (r < 0) {
-    ret = -1;
-    *entropy_used = 1;
-    r = u2p_solver_w(uu, pm, gm, 1, gam);
-    if (r < 0) ret = -2;
-  }
-  if (r >= 0) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) pp[i] = pm[i];
-  } else {
-    ret = -3;  // pp keeps the incoming primitives (ppbak)
+    ret = -3;  // pp keeps the incoming primitives
+    pp[RHO] = keep[0];
+    pp[UU] = keep[1];
+    pp[VX] = keep[2];
+    pp[VY] = keep[3];
+    pp[VZ] = keep[4];
   }
   return ret;
 }
@@ -268,9 +321,8 @@ KZD int check_floors_mhd(double *pp, const Geo &gm, double pg, const kz_floor_pa
       p2u_mhd(dpp, duu, gm, pg);
 #pragma unroll
       for (int iv = 0; iv < NV; ++iv) uu[iv] = iv <= B3 ? uu_entry[iv] + duu[iv] : 0.0;
-      int rt = u2p_solver_w(uu, pp, gm, 0, pg);
-      if (rt < 0) rt = u2p_solver_w(uu, pp, gm, 1, pg);
-      if (rt < 0) {
+      int etype = 0;
+      if (u2p_solver_w(uu, pp, gm, &etype, true, pg) < 0) {
 #pragma unroll
         for (int iv = 0; iv < NV; ++iv) pp[iv] = pporg[iv];
         pp[RHO] *= f;
@@ -608,9 +660,8 @@ KZD int apply_constraints(double *pp, double *uu, const double *uu0, const ImpCt
   for (int k = 0; k < 4; ++k) uu[UU + k] = uu0[UU + k] - (uu[EE + k] - uu0[EE + k]);
 #pragma unroll
   for (int k = 0; k < 3; ++k) uu[B1 + k] = gdetu * pp[B1 + k];
-  int rt = u2p_solver_w(uu, pp, gm, 0, cx.gam);
-  if (rt < 0 && cx.ip->allow_entr_in_4dprim) rt = u2p_solver_w(uu, pp, gm, 1, cx.gam);
-  int ret = rt < 0 ? -2 : 0;
+  int etype = 0;
+  int ret = u2p_solver_w(uu, pp, gm, &etype, cx.ip->allow_entr_in_4dprim != 0, cx.gam) < 0 ? -2 : 0;
   double ucon[4], ucov[4];
   ucon_ucov(pp, gm, ucon, ucov);
   pp[ENTR] = s_from_u(pp[RHO], pp[UU], cx.gam);
@@ -629,14 +680,14 @@ struct LagOpac {
 };
 
 // implicit.zig:337-427 residualG (scalar) on a filled state
-template <int WP>
-KZD double residual(const double *uu, const double *pp, const RadState &st, const double *uu0, const State0 &s0,
+template <int WP, bool ALL>
+KZDM double residual(const double *uu, const double *pp, const RadState &st, const double *uu0, const State0 &s0,
                     double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
   const Geo &gm = *cx.gm;
   double gdetu = gm.gdet;
   double dtau = dt / st.ucon[0];
   double giff0, gilab[4], gi[4];
-  calc_gi(st, *cx.op, cx.opdamp, &giff0, gilab);
+  calc_gi<ALL>(st, *cx.op, cx.opdamp, &giff0, gilab);
   lower4(gilab, gm, gi);
   double err[4] = {0, 0, 0, 0};
   const double SMALLI = 1.0e-80;
@@ -646,21 +697,19 @@ KZD double residual(const double *uu, const double *pp, const RadState &st, cons
     // MHD: uu - uu0 - dt*gdet*G;  RAD: uu - uu0 + dt*gdet*G
     f[k] = (WP == WP_MHD) ? uu[base + k] - uu0[base + k] - dt * gdetu * gi[k]
                           : uu[base + k] - uu0[base + k] + dt * gdetu * gi[k];
-    err[k] = (kzm_fabs(f[k]) > SMALLI) ? kzm_fabs(f[k]) / (1.0e-20 * uu[base] + kzm_fabs(uu[base + k]) +
-                                                           kzm_fabs(uu0[base + k]) + kzm_fabs(dt * gdetu * gi[k]))
-                                       : 0.0;
+    const double e = kzm_fabs(f[k]) / (1.0e-20 * uu[base] + kzm_fabs(uu[base + k]) + kzm_fabs(uu0[base + k]) +
+                                       kzm_fabs(dt * gdetu * gi[k]));
+    err[k] = dm_sel(kzm_fabs(f[k]) > SMALLI, e, 0.0);
   }
   if (wf == WF_LAB) {
     if (WP == WP_RAD) {
       f[0] = uu[EE] - uu0[EE] + dt * gdetu * gi[0];
-      err[0] = (kzm_fabs(f[0]) > SMALLI)
-                   ? kzm_fabs(f[0]) / (kzm_fabs(uu[EE]) + kzm_fabs(uu0[EE]) + kzm_fabs(dt * gdetu * gi[0]))
-                   : 0.0;
+      const double e = kzm_fabs(f[0]) / (kzm_fabs(uu[EE]) + kzm_fabs(uu0[EE]) + kzm_fabs(dt * gdetu * gi[0]));
+      err[0] = dm_sel(kzm_fabs(f[0]) > SMALLI, e, 0.0);
     } else {
       f[0] = uu[UU] - uu0[UU] - dt * gdetu * gi[0];
-      err[0] = (kzm_fabs(f[0]) > SMALLI)
-                   ? kzm_fabs(f[0]) / (kzm_fabs(uu[UU]) + kzm_fabs(uu0[UU]) + kzm_fabs(dt * gdetu * gi[0]))
-                   : 0.0;
+      const double e = kzm_fabs(f[0]) / (kzm_fabs(uu[UU]) + kzm_fabs(uu0[UU]) + kzm_fabs(dt * gdetu * gi[0]));
+      err[0] = dm_sel(kzm_fabs(f[0]) > SMALLI, e, 0.0);
     }
   } else if (we == WE_ENERGY) {
     if (WP == WP_RAD) {
@@ -685,46 +734,57 @@ KZD double residual(const double *uu, const double *pp, const RadState &st, cons
 // fills the state right after each applyConstraints and consumes it only
 // here, with pp unchanged in between, so filling at the point of use gives
 // the same values and keeps the state a temporary.
-template <int WP>
-KZD double eval_residual(const double *uu, const double *pp, const LagOpac &lag, const double *uu0,
-                         const State0 &s0, double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
+template <int WP, bool ALL>
+KZDM double eval_residual_t(const double *uu, const double *pp, const LagOpac &lag, const double *uu0,
+                            const State0 &s0, double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
   RadState st;
-  fill_radstate(pp, *cx.gm, cx.gam, *cx.op, we == WE_ENTROPY, st);
+  fill_radstate_t<ALL>(pp, *cx.gm, cx.gam, *cx.op, we == WE_ENTROPY, st);
   if (cx.ip->lag_opac) {
     st.kappaes = lag.kappaes;
     st.op = lag.op;
   }
-  return residual<WP>(uu, pp, st, uu0, s0, dt, cx, we, wf, f);
+  return residual<WP, ALL>(uu, pp, st, uu0, s0, dt, cx, we, wf, f);
+}
+template <int WP>
+KZDM double eval_residual(const double *uu, const double *pp, const LagOpac &lag, const double *uu0,
+                          const State0 &s0, double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
+  return all_channels(*cx.op) ? eval_residual_t<WP, true>(uu, pp, lag, uu0, s0, dt, cx, we, wf, f)
+                              : eval_residual_t<WP, false>(uu, pp, lag, uu0, s0, dt, cx, we, wf, f);
 }
 
 // implicit.zig:431-467 f1dErr (energy equation, undamped opacities)
-KZD double f1d_err(double xxx, const double *pp0, double dtau, const ImpCtx &cx, int wp, double totenergy,
-                   double ratio) {
-  double ugas, ehat;
-  if (wp == WP_RAD) {
-    ehat = xxx * ratio;
-    ugas = totenergy - ehat;
-  } else {
-    ugas = xxx;
-    ehat = totenergy - ugas;
-  }
+template <bool ALL>
+KZDM double f1d_err_t(double xxx, const double *pp0, double dtau, const ImpCtx &cx, int wp, double totenergy,
+                      double ratio) {
+  const bool rad = wp == WP_RAD;
+  const double xr = xxx * ratio;
+  const double ehat = dm_sel(rad, xr, totenergy - xxx);
+  const double ugas = dm_sel(rad, totenergy - xr, xxx);
   double pp[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) pp[i] = pp0[i];
   pp[UU] = ugas;
   pp[EE] = ehat / ratio;
   RadState st;
-  fill_radstate(pp, *cx.gm, cx.gam, *cx.op, false, st);
+  fill_radstate_t<ALL>(pp, *cx.gm, cx.gam, *cx.op, false, st);
   double giff0, gilab[4];
-  calc_gi(st, *cx.op, cx.op->opdamp, &giff0, gilab);
-  if (wp == WP_RAD) return ehat - pp0[EE] / ratio + dtau * giff0;
-  return ugas - pp0[UU] - dtau * giff0;
+  calc_gi<ALL>(st, *cx.op, cx.op->opdamp, &giff0, gilab);
+  return dm_sel(rad, ehat - pp0[EE] / ratio + dtau * giff0, ugas - pp0[UU] - dtau * giff0);
+}
+KZDM double f1d_err(double xxx, const double *pp0, double dtau, const ImpCtx &cx, int wp, double totenergy,
+                    double ratio) {
+  return all_channels(*cx.op) ? f1d_err_t<true>(xxx, pp0, dtau, cx, wp, totenergy, ratio)
+                              : f1d_err_t<false>(xxx, pp0, dtau, cx, wp, totenergy, ratio);
 }
 
 // implicit.zig:473-574 solve1dPrim: bisection warm start on the fluid-frame
-// energy equation; reads Ehat, u^t and T_gas of the reference state.
-KZD void solve_1d_prim(const double *pp00, double st_ehat, double st_ut, double st_tgas, double dt, const ImpCtx &cx,
-                       double *pp0out) {
+// energy equation; reads Ehat, u^t and T_gas of the reference state.  The
+// reference evaluates the equation in four places (both ends of the bracket,
+// its growth, the midpoints); here they are one loop with one evaluation, so
+// that its code stands once and the lanes of a wave share it wherever each of
+// them is.
+KZDM void solve_1d_prim(const double *pp00, double st_ehat, double st_ut, double st_tgas, double dt, const ImpCtx &cx,
+                        double *pp0out) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) pp0out[i] = pp00[i];
   double ehat = st_ehat;
@@ -747,133 +807,215 @@ KZD void solve_1d_prim(const double *pp00, double st_ehat, double st_ut, double 
     xlo = pe / 1.05;
     xhi = kzm_fmin(pe * 1.05, (pe + fac * tot / ratio) / fac1);
   }
-  double elo = f1d_err(xlo, pp00, dtau, cx, wp, tot, ratio);
-  double ehi = f1d_err(xhi, pp00, dtau, cx, wp, tot, ratio);
-  int iter = 0;
-  while (elo * ehi > 0.0) {
-    iter += 1;
-    if (elo > 0.0) {
-      xhi = xlo;
-      ehi = elo;
-      xlo /= fac;
-      elo = f1d_err(xlo, pp00, dtau, cx, wp, tot, ratio);
-    } else {
-      xlo = xhi;
-      elo = ehi;
-      if (wp == WP_RAD) xhi = kzm_fmin(xhi * fac, (xhi + fac * tot / ratio) / fac1);
-      else xhi = kzm_fmin(xhi * fac, (xhi + fac * tot) / fac1);
-      ehi = f1d_err(xhi, pp00, dtau, cx, wp, tot, ratio);
-    }
-    if (elo != elo || ehi != ehi) iter = 50;
-    if (iter >= 50) break;
-  }
-  if (iter >= 50) return;
-  double xmid;
+  enum { LOW, HIGH, GROW_LOW, GROW_HIGH, MID };
+  int at = LOW, iter = 0;
+  double elo = 0, ehi = 0, x = xlo;
   for (;;) {
-    iter += 1;
-    xmid = 0.5 * (xlo + xhi);
-    double emid = f1d_err(xmid, pp00, dtau, cx, wp, tot, ratio);
-    if (emid * elo > 0.0) {
-      xlo = xmid;
-      elo = emid;
-    } else {
-      xhi = xmid;
-      ehi = emid;
+    const double e = f1d_err(x, pp00, dtau, cx, wp, tot, ratio);
+    if (at == LOW) {
+      elo = e;
+      x = xhi;
+      at = HIGH;
+      continue;
     }
-    if (xmid != xmid || emid != emid) return;
-    if (!(kzm_fabs((xhi - xlo) / xmid) > 1.0e-3)) break;
+    if (at == MID) {
+      if (e * elo > 0.0) {
+        xlo = x;
+        elo = e;
+      } else {
+        xhi = x;
+        ehi = e;
+      }
+      if (x != x || e != e) return;
+      if (!(kzm_fabs((xhi - xlo) / x) > 1.0e-3)) break;
+    } else {
+      if (at == GROW_LOW) elo = e;
+      else ehi = e;
+      if (at != HIGH && (elo != elo || ehi != ehi)) iter = 50;
+      if (iter >= 50) return;
+      if (elo * ehi > 0.0) {
+        iter += 1;
+        if (elo > 0.0) {
+          xhi = xlo;
+          ehi = elo;
+          xlo /= fac;
+          x = xlo;
+          at = GROW_LOW;
+        } else {
+          xlo = xhi;
+          elo = ehi;
+          if (wp == WP_RAD) xhi = kzm_fmin(xhi * fac, (xhi + fac * tot / ratio) / fac1);
+          else xhi = kzm_fmin(xhi * fac, (xhi + fac * tot) / fac1);
+          x = xhi;
+          at = GROW_HIGH;
+        }
+        continue;
+      }
+    }
+    at = MID;
+    x = 0.5 * (xlo + xhi);
   }
   if (wp == WP_RAD) {
-    pp0out[EE] = xmid;
-    pp0out[UU] = tot - xmid * ratio;
+    pp0out[EE] = x;
+    pp0out[UU] = tot - x * ratio;
   } else {
-    pp0out[UU] = xmid;
-    pp0out[EE] = (tot - xmid) / ratio;
+    pp0out[UU] = x;
+    pp0out[EE] = (tot - x) / ratio;
   }
 }
 
 // Element j (0..3, not a compile-time constant) of a 4-block, by selects,
 // so that register-resident arrays are never indexed dynamically.
-KZD double get4(const double *a, int j) { return j == 0 ? a[0] : (j == 1 ? a[1] : (j == 2 ? a[2] : a[3])); }
-KZD void set4(double *a, int j, double v) {
-  if (j == 0) a[0] = v;
-  else if (j == 1) a[1] = v;
-  else if (j == 2) a[2] = v;
-  else a[3] = v;
+// (the values are taken before the choice: a choice between addresses would
+// keep the array, and the whole structure around it, in scratch memory)
+KZDM double get4(const double *a, int j) {
+  const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+  return j == 0 ? a0 : (j == 1 ? a1 : (j == 2 ? a2 : a3));
 }
-KZD double gdiag(const Geo &gm, int j) { return j == 1 ? gm.g[1][1] : (j == 2 ? gm.g[2][2] : gm.g[3][3]); }
+KZDM void set4(double *a, int j, double v) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = j == k ? v : a[k];
+}
+KZDM double gdiag(const Geo &gm, int j) {
+  const double g1 = gm.g[1][1], g2 = gm.g[2][2], g3 = gm.g[3][3];
+  return j == 1 ? g1 : (j == 2 ? g2 : g3);
+}
 
 // implicit.zig:586-591 fdDel on the block b = ppp + sh
-KZD double fd_del(int j, double sign, const double *b, double eps, const Geo &gm) {
+KZDM double fd_del(int j, double sign, const double *b, double eps, const Geo &gm) {
   if (j == 0) return sign * eps * b[0];
   double bj = get4(b, j);
   double veleps = eps * my_sign(bj) * kzm_fmax(1.0e-8 / kzm_sqrt(gdiag(gm, j)), kzm_fabs(bj));
   return bj >= 0.0 ? sign * veleps : -sign * veleps;
 }
 
-// implicit.zig:642-922 solve4dPrimCore (scalar Jacobian), as a start and a
-// one-iteration step so that a persistent kernel can interleave cells at
-// different iterations: newton_step runs one pass of the reference's
-// iteration loop and returns 0 to go on, 1 when the loop ends solved (n.pp
-// and n.iter hold the result) and -1 when it ends failed.
+// implicit.zig:642-922 solve4dPrimCore (scalar Jacobian) as a start and a
+// pass that evaluates one trial state: newton_pass applies the constraints to
+// n.pp, judges them by what the state was tried for (n.at: the base of an
+// iteration, one column of the Jacobian, or the update), takes the residual
+// there and sets up the next trial state.  It returns 0 to go on, 1 when the
+// reference's loop ends solved (n.pp and n.iter hold the result) and -1 when
+// it ends failed; the sequence of trial states is the reference's.
+//
+// One pass per trial state, so that the constraints and the residual stand in
+// the code once each.  Written out per use (three and two copies per
+// primitive block) the first rung's code was 293 KB (145 KB now) against the
+// 64 KB of instruction cache that two CUs share, with 400 B of scratch per
+// lane (none now).  It also lets the lanes of a wave stand at different trial
+// states.  First rung at 384x360, with kz_dev_math.h: 262 -> 194 us.
+enum { AT_BASE = 0, AT_COL, AT_UPDATE };
 struct NewtonState {
   double uu[NV], pp[NV];
-  int iter, fret;
+  double b[4];        // the iteration's primitive block
+  double rho0, en0;   // its density, and the energy density of the other block
+  double f1[4];       // residual at the base
+  double jac[4][4];   // Jacobian, then the scaled inverse that the update applies
+  double errbase, del, xiapp;
+  int iter, at, j;
+  bool second;        // the column's second sign
 };
 template <int WP>
-KZD void newton_start(NewtonState &n, const double *uu00, const double *pp0in, const ImpCtx &cx) {
+KZD void newton_start(NewtonState &n, const double *uu00, const double *pp0in) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     n.uu[i] = uu00[i];
     n.pp[i] = pp0in[i];
   }
-  n.fret = apply_constraints<WP>(n.pp, n.uu, uu00, cx);
   n.iter = 0;
+  n.at = AT_BASE;
+}
+// the update's trial state ppp - xiapp * (inverse) * f1
+KZDM void newton_update(NewtonState &n, double *blk) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    double x = n.b[i];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x -= n.xiapp * n.jac[i][j] * n.f1[j];
+    blk[i] = x;
+  }
 }
 template <int WP>
-KZD int newton_step(NewtonState &n, const double *uu00, const LagOpac &lag, const State0 &s0, double dt,
+KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, const State0 &s0, double dt,
                     const ImpCtx &cx, int we, int wf) {
   const kz_implicit_params &ip = *cx.ip;
   const Geo &gm = *cx.gm;
   double *uu = n.uu, *pp = n.pp;
-  double ppp[NV];
   constexpr int sh = (WP == WP_MHD) ? UU : EE;
-  const double conv = (we == WE_ENTROPY) ? ip.entrconv : ip.conv;
-  double f1[4], f2[4], jac[4][4];
-  bool failed = false;
-  int &fret = n.fret;
-  const int iter = ++n.iter;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) ppp[i] = pp[i];
-  if (fret < -1) return -1;
-  double errbase = eval_residual<WP>(uu, pp, lag, uu00, s0, dt, cx, we, wf, f1);
-  if (errbase < conv) return iter > ip.maxiter ? -1 : 1;
-#pragma unroll 1
-  for (int j = 0; j < 4; ++j) {
-    double sign = -1.0;
-    for (;;) {
-      double del = fd_del(j, sign, ppp + sh, ip.eps, gm);
-      set4(pp + sh, j, get4(ppp + sh, j) + del);
-      fret = apply_constraints<WP>(pp, uu, uu00, cx);
-      if (fret < -1) {
-        if (sign > 0.0) {
-          failed = true;
-          break;
-        }
-        set4(pp + sh, j, get4(ppp + sh, j));
-        sign *= -1.0;
-        continue;
+  constexpr int other = (WP == WP_MHD) ? EE : UU;
+  double *blk = pp + sh;
+  const int fret = apply_constraints<WP>(pp, uu, uu00, cx);
+  if (n.at == AT_UPDATE) {
+    bool ok = false;
+    double edenmin = n.b[0] / ip.max_en_change_down;
+    double edenmax = n.b[0] * ip.max_en_change_up;
+    if (blk[0] > edenmin && blk[0] < edenmax && fret >= -1) ok = true;
+    double tgo = t_from_urho(*cx.op, WP == WP_MHD ? n.b[0] : n.en0, n.rho0, cx.gam);
+    double tgn = t_from_urho(*cx.op, pp[UU], pp[RHO], cx.gam);
+    if (ok && (tgn > tgo * ip.max_tgas_change || tgn < tgo / ip.max_tgas_change)) ok = false;
+    double trn = lte_t_from_e(*cx.op, pp[EE]);
+    double tro = lte_t_from_e(*cx.op, WP == WP_MHD ? n.en0 : n.b[0]);
+    if (ok && (trn > tro * ip.max_trad_change || trn < tro / ip.max_trad_change)) ok = false;
+    if (!ok) {
+      if (blk[0] <= 0.0) {
+        n.xiapp *= n.b[0] / (n.b[0] + kzm_fabs(blk[0]));
+        n.xiapp *= 1.0e-1;
+      } else {
+        n.xiapp /= ip.damping_factor;
       }
-      eval_residual<WP>(uu, pp, lag, uu00, s0, dt, cx, we, wf, f2);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) set4(jac[i], j, (f2[i] - f1[i]) / del);
-      set4(pp + sh, j, get4(ppp + sh, j));
-      break;
+      if (n.xiapp < ip.max_damping) return -1;
+      newton_update(n, blk);
+      return 0;
     }
-    if (failed) break;
+    double f3[4];
+    f3[0] = kzm_fabs((blk[0] - n.b[0]) / n.b[0]);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) f3[i] = kzm_fabs((blk[i] - n.b[i]) / kzm_fmax(ip.eps, kzm_fabs(n.b[i])));
+    double cr = (we == WE_ENTROPY) ? ip.convrelentr : ip.convrel;
+    double cre = (we == WE_ENTROPY) ? ip.convrelentrerr : ip.convrelerr;
+    bool cc = true;
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+      if (f3[ib] > cr) cc = false;
+    if (cc || n.errbase <= cre) return n.iter > ip.maxiter ? -1 : 1;
+    if (n.iter > ip.maxiter) return -1;
+    n.at = AT_BASE;
+  } else if (fret < -1) {
+    if (n.at == AT_BASE || n.second) return -1;
+    n.second = true;
+    set4(blk, n.j, get4(n.b, n.j));
+    n.del = fd_del(n.j, 1.0, n.b, ip.eps, gm);
+    set4(blk, n.j, get4(n.b, n.j) + n.del);
+    return 0;
   }
-  if (failed) return -1;
-  double sv[4] = {pp[sh], 1.0, 1.0, 1.0}, isv[4];
+  double f[4];
+  const double err = eval_residual<WP>(uu, pp, lag, uu00, s0, dt, cx, we, wf, f);
+  if (n.at == AT_BASE) {
+    n.iter += 1;
+    const double conv = (we == WE_ENTROPY) ? ip.entrconv : ip.conv;
+    if (err < conv) return n.iter > ip.maxiter ? -1 : 1;
+    n.errbase = err;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      n.b[i] = blk[i];
+      n.f1[i] = f[i];
+    }
+    n.rho0 = pp[RHO];
+    n.en0 = pp[other];
+    n.at = AT_COL;
+    n.j = 0;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) set4(n.jac[i], n.j, (f[i] - n.f1[i]) / n.del);
+    set4(blk, n.j, get4(n.b, n.j));
+    n.j += 1;
+  }
+  if (n.j < 4) {
+    n.second = false;
+    n.del = fd_del(n.j, -1.0, n.b, ip.eps, gm);
+    set4(blk, n.j, get4(n.b, n.j) + n.del);
+    return 0;
+  }
+  double sv[4] = {blk[0], 1.0, 1.0, 1.0}, isv[4];
   if (ip.scale_jacobian) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -889,7 +1031,7 @@ KZD int newton_step(NewtonState &n, const double *uu00, const LagOpac &lag, cons
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) jf[i][j] = (float)jac[i][j];
+      for (int j = 0; j < 4; ++j) jf[i][j] = (float)n.jac[i][j];
     if (ip.scale_jacobian) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -908,75 +1050,28 @@ KZD int newton_step(NewtonState &n, const double *uu00, const LagOpac &lag, cons
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (i != j) jac[i][j] = jac[i][j] * (sv[j] * isv[i]);
+          if (i != j) n.jac[i][j] = n.jac[i][j] * (sv[j] * isv[i]);
     }
-    invert4(jac, ij);
+    invert4(n.jac, ij);
   }
-  double xiapp = 1.0;
-  double xxx[4];
-  for (;;) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) xxx[k] = ppp[k + sh];
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (ip.scale_jacobian) xxx[i] -= xiapp * (ij[i][j] * sv[i] * isv[j]) * f1[j];
-        else xxx[i] -= xiapp * ij[i][j] * f1[j];
-      }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pp[k + sh] = xxx[k];
-    fret = apply_constraints<WP>(pp, uu, uu00, cx);
-    bool ok = false;
-    double edenmin = ppp[sh] / ip.max_en_change_down;
-    double edenmax = ppp[sh] * ip.max_en_change_up;
-    if (xxx[0] > edenmin && xxx[0] < edenmax && fret >= -1) ok = true;
-    double tgo = t_from_urho(*cx.op, ppp[UU], ppp[RHO], cx.gam);
-    double tgn = t_from_urho(*cx.op, pp[UU], pp[RHO], cx.gam);
-    if (ok && (tgn > tgo * ip.max_tgas_change || tgn < tgo / ip.max_tgas_change)) ok = false;
-    double trn = lte_t_from_e(*cx.op, pp[EE]);
-    double tro = lte_t_from_e(*cx.op, ppp[EE]);
-    if (ok && (trn > tro * ip.max_trad_change || trn < tro / ip.max_trad_change)) ok = false;
-    if (ok) break;
-    if (xxx[0] <= 0.0) {
-      xiapp *= ppp[sh] / (ppp[sh] + kzm_fabs(xxx[0]));
-      xiapp *= 1.0e-1;
-    } else {
-      xiapp /= ip.damping_factor;
-    }
-    if (xiapp < ip.max_damping) {
-      failed = true;
-      break;
-    }
-  }
-  if (!failed) {
-    double f3[4];
-    f3[0] = kzm_fabs((pp[sh] - ppp[sh]) / ppp[sh]);
-#pragma unroll
-    for (int i = 1; i < 4; ++i) {
-      double d = pp[i + sh] - ppp[i + sh];
-      f3[i] = kzm_fabs(d / kzm_fmax(ip.eps, kzm_fabs(ppp[i + sh])));
-    }
-    double cr = (we == WE_ENTROPY) ? ip.convrelentr : ip.convrel;
-    double cre = (we == WE_ENTROPY) ? ip.convrelentrerr : ip.convrelerr;
-    bool cc = true;
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-      if (f3[ib] > cr) cc = false;
-    if (cc || errbase <= cre) return iter > ip.maxiter ? -1 : 1;
-  }
-  if (iter > ip.maxiter || failed) return -1;
+    for (int j = 0; j < 4; ++j) n.jac[i][j] = ip.scale_jacobian ? ij[i][j] * sv[i] * isv[j] : ij[i][j];
+  n.xiapp = 1.0;
+  n.at = AT_UPDATE;
+  newton_update(n, blk);
   return 0;
 }
 template <int WP>
-__device__ static __forceinline__ bool solve_4d_prim_core(const double *uu00, const LagOpac &lag, const State0 &s0,
+KZDM bool solve_4d_prim_core(const double *uu00, const LagOpac &lag, const State0 &s0,
                                                           const double *pp0in, double dt, const ImpCtx &cx, int we,
                                                           int wf, double *pp_out, int *iters_out) {
   NewtonState n;
-  newton_start<WP>(n, uu00, pp0in, cx);
+  newton_start<WP>(n, uu00, pp0in);
   int r;
   do {
-    r = newton_step<WP>(n, uu00, lag, s0, dt, cx, we, wf);
+    r = newton_pass<WP>(n, uu00, lag, s0, dt, cx, we, wf);
   } while (r == 0);
   if (r < 0) return false;
 #pragma unroll

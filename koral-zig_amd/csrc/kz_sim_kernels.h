@@ -720,7 +720,7 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
           s.geo(t, gm);
           dt = s.dt(t);
           const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-          newton_start<WP>(ns, uu00, pp0, cx);
+          newton_start<WP>(ns, uu00, pp0);
           has = true;
         }
       }
@@ -729,7 +729,7 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
     if (!__ballot(has)) break;
     if (has) {
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-      const int r = newton_step<WP>(ns, uu00, lag, s0, dt, cx, we, wf);
+      const int r = newton_pass<WP>(ns, uu00, lag, s0, dt, cx, we, wf);
       if (r != 0) {
         done(t, gm, ns, r > 0);
         has = false;
@@ -803,8 +803,8 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
       int r = -1;
       if (ir > 0) {
-        r = (wp == WP_MHD) ? newton_step<WP_MHD>(ns, uu00, lag, s0, dt, cx, we, wf)
-                           : newton_step<WP_RAD>(ns, uu00, lag, s0, dt, cx, we, wf);
+        r = (wp == WP_MHD) ? newton_pass<WP_MHD>(ns, uu00, lag, s0, dt, cx, we, wf)
+                           : newton_pass<WP_RAD>(ns, uu00, lag, s0, dt, cx, we, wf);
       }
       if (r > 0) {
         s.solved(ph, t, gm, ns.pp, ns.iter, ir, wp, we, wf);
@@ -820,8 +820,8 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
           wp = (ir == 1 || ir == 4) ? sw : ot;
           we = (ir >= 4) ? WE_ENTROPY : WE_ENERGY;
           wf = (ir == 2) ? WF_LAB : WF_FF;
-          if (wp == WP_MHD) newton_start<WP_MHD>(ns, uu00, pp0, cx);
-          else newton_start<WP_RAD>(ns, uu00, pp0, cx);
+          if (wp == WP_MHD) newton_start<WP_MHD>(ns, uu00, pp0);
+          else newton_start<WP_RAD>(ns, uu00, pp0);
         }
       }
     }
