@@ -914,8 +914,7 @@ struct NewtonState {
   int iter, at, j;
   bool second;        // the column's second sign
 };
-template <int WP>
-KZD void newton_start(NewtonState &n, const double *uu00, const double *pp0in) {
+KZDM void newton_start(NewtonState &n, const double *uu00, const double *pp0in) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     n.uu[i] = uu00[i];
@@ -1068,7 +1067,7 @@ KZDM bool solve_4d_prim_core(const double *uu00, const LagOpac &lag, const State
                                                           const double *pp0in, double dt, const ImpCtx &cx, int we,
                                                           int wf, double *pp_out, int *iters_out) {
   NewtonState n;
-  newton_start<WP>(n, uu00, pp0in);
+  newton_start(n, uu00, pp0in);
   int r;
   do {
     r = newton_pass<WP>(n, uu00, lag, s0, dt, cx, we, wf);

@@ -58,6 +58,7 @@ struct Dev {
   int32_t *imp_rl;                // [2][nd] cells the persistent first rung left
   unsigned long long *imp_rc;     // [2] their lengths
   unsigned long long *imp_qpos;   // [3] queue claim positions
+  unsigned *imp_st;               // [nd] rungs that have failed or solved a cell
   // the u2p fixup list
   unsigned *sync;     // [SY_NFIX] u2p fixup list length
   int32_t *fix_list;  // domain cells flagged for a u2p fixup

@@ -407,6 +407,7 @@ struct ImpWork {
   int32_t *rl;
   unsigned long long *rc;
   unsigned long long *qpos;
+  unsigned *st;  // [n] by cell: which rungs past the first have failed or solved it
 };
 // The cells of one run's domain (opImplicit, sim.zig:1736-1776): polar rows
 // are skipped, dt is a step scalar, a solved cell stores u and p and clears
@@ -679,8 +680,18 @@ struct RungDone {
     const long nd = s->count();
     unsigned long long k = atomicAdd(&w->rc[which], 1ULL);
     w->rl[which * nd + k] = (int32_t)t;
+    w->st[t] = 0;
   }
 };
+// Lanes of a wave that take cells from a queue of qlen entries.  Where the
+// entries do not fill the launch, they are spread over its waves rather than
+// packed 64 to a wave: lanes at different depths of their solves run one
+// after the other, and a wave of its own costs an idle SIMD nothing (4099
+// cells: first rung 15 -> 7 ms per solve).
+__device__ __forceinline__ int queue_lanes(long qlen) {
+  const long per = (qlen + gridDim.x - 1) / gridDim.x;
+  return per < 1 ? 1 : (per > 64 ? 64 : (int)per);
+}
 // Work stealing over one queue (cells list[0 .. qlen)) with Newton variant
 // WP at opdamp level 0: each lane holds one cell; the lanes without one claim
 // the next queue entries together (one atomic per wave and refill) until the
@@ -693,7 +704,7 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ULL << lane) - 1ULL;
   const long nd = s.count();
-  bool has = false, exhausted = qlen <= 0;
+  bool has = false, exhausted = qlen <= 0 || lane >= queue_lanes(qlen);
   long t = 0;
   double dt = 0;
   NewtonState ns;
@@ -720,13 +731,16 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
           s.geo(t, gm);
           dt = s.dt(t);
           const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-          newton_start<WP>(ns, uu00, pp0);
+          newton_start(ns, uu00, pp0);
           has = true;
         }
       }
-      if (base + cnt >= qlen) exhausted = true;  // the same for every lane of the wave
+      if (base + cnt >= qlen) exhausted = true;
     }
-    if (!__ballot(has)) break;
+    if (!__ballot(has)) {
+      if (__ballot(!exhausted)) continue;
+      break;
+    }
     if (has) {
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
       const int r = newton_pass<WP>(ns, uu00, lag, s0, dt, cx, we, wf);
@@ -747,27 +761,51 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_rung0_persist(S
   const RungDone<S> dm{&s, &w, &ph, 0, 0, WP_MHD, WE_ENERGY, WF_LAB};
   drain_queue<S, WP_MHD>(s, w, ph, w.list, n_mhd(w), &w.qpos[1], WE_ENERGY, WF_LAB, dm);
 }
-// Rungs 1..5 of level 0 (implicit.zig:961-968) over the cells the first
-// rung left (both starting-block lists, MHD start then RAD start), work
-// stealing as drain_queue but with each lane walking its own cell up the
-// ladder: when an attempt fails the lane starts the next rung's Newton (whose
-// primitive block may differ from its neighbours', the two variants then run
-// one after the other), so the long ladders of different rungs overlap
-// instead of each rung waiting for its slowest cell.  Cells past rung 5 go
-// to the slow list.
+// bits of ImpWork::st: RUNG_FAILED << r and RUNG_SOLVED << r for rung r = 1..5
+constexpr unsigned RUNG_FAILED = 1u, RUNG_SOLVED = 1u << 8, RUNG_FAILED_MASK = 0x3eu;
+// a cell's bits as the other waves have set them (past this die's caches)
+__device__ __forceinline__ unsigned rung_state(const ImpWork &w, long t) {
+  return __hip_atomic_load(&w.st[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool rung_solved_below(const ImpWork &w, long t, int ir) {
+  return rung_state(w, t) & (((1u << ir) - 2u) * RUNG_SOLVED);
+}
+// Rungs 1..5 of level 0 (implicit.zig:961-968) over the m cells the first
+// rung left (both starting-block lists, MHD start then RAD start), as one
+// queue of 5 m attempts ordered by rung.  Every attempt starts from the stored
+// reference state and knows nothing of the others, so the rungs of a cell may
+// run at the same time; the cell takes the solution of the lowest rung that
+// solves it, as the reference's ladder does.  w.st[cell] has a bit for each
+// rung that failed and one for each that solved:
+//   a lane whose attempt solved its cell stores the solution once every lower
+//   rung has failed, waits while some are open, and drops it when one solves;
+//   an attempt that is under way or about to start is dropped when a lower
+//   rung has solved the cell;
+//   the attempt that completes five failures sends the cell to the slow list.
+// A lane waits only for attempts that were claimed before its own and that
+// their lanes began at once, each at most maxiter + 1 iterations long, so
+// every wave ends.  Attempts of one rung and starting block stand together in
+// the queue, so a wave's lanes mostly run one primitive block.
+//
+// Bound by the serial chain of the longest ladder: run one after the other by
+// one lane per cell, the five rungs of the slowest cell set the time of every
+// batch.  Per solve, with queue_lanes: 59 -> 9 ms at 4099 cells (480 of them
+// here), 148 -> 49 ms at 2^19.  In the independent-cell batch rung 1 fails for 93 % of these cells and rung 2 then
+// solves 96 %, so little is tried in vain.
 template <class S, bool BR>
 __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(S s, ImpWork w, kz_physics ph) {
   ph.opac.synchrotron_bridge = BR;
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ULL << lane) - 1ULL;
   const long nd = s.count();
-  const long n0 = (long)w.rc[0], qlen = n0 + (long)w.rc[1];
-  bool has = false, exhausted = qlen <= 0;
+  const long n0 = (long)w.rc[0], m = n0 + (long)w.rc[1], qlen = 5 * m;
+  // lanes for the two rungs that most of these cells need
+  bool has = false, held = false, exhausted = qlen <= 0 || lane >= queue_lanes(2 * m);
   long t = 0;
-  int sw = WP_MHD, ir = 1, wp = WP_MHD, we = WE_ENERGY, wf = WF_FF;
+  int ir = 1, wp = WP_MHD, we = WE_ENERGY, wf = WF_FF;
   double dt = 0;
   NewtonState ns;
-  double uu00[NV], pp0[NV];
+  double uu00[NV];
   State0 s0;
   LagOpac lag;
   Geo gm;
@@ -782,49 +820,61 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
       if (!has && !exhausted) {
         const long q = base + __popcll(need & below);
         if (q < qlen) {
-          sw = q < n0 ? WP_MHD : WP_RAD;
-          t = q < n0 ? w.rl[q] : w.rl[nd + (q - n0)];
+          ir = 1 + (int)(q / m);
+          const long i = q - (ir - 1) * m;
+          const int sw = i < n0 ? WP_MHD : WP_RAD, ot = i < n0 ? WP_RAD : WP_MHD;
+          t = i < n0 ? w.rl[i] : w.rl[nd + (i - n0)];
           if (ph.implicit.opdamp_maxlevels < 0) {  // no level to run (implicit.zig:961)
-            unsigned long long k = atomicAdd(w.nslow, 1ULL);
-            w.slow[k] = (int32_t)t;
-          } else {
+            if (ir == 1) {
+              unsigned long long k = atomicAdd(w.nslow, 1ULL);
+              w.slow[k] = (int32_t)t;
+            }
+          } else if (!rung_solved_below(w, t, ir)) {
+            double pp0[NV];
             imp_load(w, nd, t, uu00, pp0, s0, lag);
             s.geo(t, gm);
             dt = s.dt(t);
-            ir = 0;  // the next attempt is rung 1
+            wp = (ir == 1 || ir == 4) ? sw : ot;
+            we = (ir >= 4) ? WE_ENTROPY : WE_ENERGY;
+            wf = (ir == 2) ? WF_LAB : WF_FF;
+            newton_start(ns, uu00, pp0);
             has = true;
           }
         }
       }
-      if (base + cnt >= qlen) exhausted = true;  // the same for every lane of the wave
+      if (base + cnt >= qlen) exhausted = true;
     }
-    if (!__ballot(has)) break;
-    if (has) {
+    if (!__ballot(has)) {
+      if (__ballot(!exhausted)) continue;  // only attempts that nobody needs any more were claimed
+      break;
+    }
+    if (has && !held) {
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-      int r = -1;
-      if (ir > 0) {
-        r = (wp == WP_MHD) ? newton_pass<WP_MHD>(ns, uu00, lag, s0, dt, cx, we, wf)
-                           : newton_pass<WP_RAD>(ns, uu00, lag, s0, dt, cx, we, wf);
-      }
+      const int r = (wp == WP_MHD) ? newton_pass<WP_MHD>(ns, uu00, lag, s0, dt, cx, we, wf)
+                                   : newton_pass<WP_RAD>(ns, uu00, lag, s0, dt, cx, we, wf);
       if (r > 0) {
-        s.solved(ph, t, gm, ns.pp, ns.iter, ir, wp, we, wf);
-        has = false;
+        atomicOr(&w.st[t], RUNG_SOLVED << ir);
+        held = true;
       } else if (r < 0) {
-        if (ir == 5) {
+        const unsigned now = atomicOr(&w.st[t], RUNG_FAILED << ir) | (RUNG_FAILED << ir);
+        if ((now & RUNG_FAILED_MASK) == RUNG_FAILED_MASK) {
           unsigned long long k = atomicAdd(w.nslow, 1ULL);
           w.slow[k] = (int32_t)t;
-          has = false;
-        } else {  // the next rung's attempt from the stored reference state
-          ir += 1;
-          const int ot = (sw == WP_RAD) ? WP_MHD : WP_RAD;
-          wp = (ir == 1 || ir == 4) ? sw : ot;
-          we = (ir >= 4) ? WE_ENTROPY : WE_ENERGY;
-          wf = (ir == 2) ? WF_LAB : WF_FF;
-          if (wp == WP_MHD) newton_start<WP_MHD>(ns, uu00, pp0);
-          else newton_start<WP_RAD>(ns, uu00, pp0);
         }
+        has = false;
       }
     }
+    if (has && (held || ns.at == AT_UPDATE)) {
+      const unsigned now = rung_state(w, t);
+      const unsigned low = (1u << ir) - 2u;  // the rungs 1 .. ir - 1
+      if (now & (low * RUNG_SOLVED)) {
+        has = held = false;
+      } else if (held && (now & low) == low) {
+        s.solved(ph, t, gm, ns.pp, ns.iter, ir, wp, we, wf);
+        has = held = false;
+      }
+    }
+    if (!__ballot(has && !held)) __builtin_amdgcn_s_sleep(8);
   }
 }
 
@@ -882,7 +932,7 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
   const unsigned nb = nblk(n, 64);
   k_imp_prep<S, BR><<<nb, 64, 0, st>>>(cells, w, ph);
   if (persist) {
-    const unsigned np = persist_blocks < nb + 1 ? persist_blocks : nb + 1;
+    const unsigned np = persist_blocks < (unsigned long)n ? persist_blocks : (unsigned)n;
     k_imp_rung0_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_ladder_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 1);

@@ -1529,6 +1529,7 @@ kz_sim *kz_sim_create(const kz_grid *gr, const kz_physics *ph, const double *g, 
   first_err(e, dalloc(s, (void **)&D.imp_rl, (size_t)2 * nd * sizeof(int32_t)));
   first_err(e, dalloc(s, (void **)&D.imp_rc, 2 * sizeof(unsigned long long)));
   first_err(e, dalloc(s, (void **)&D.imp_qpos, 3 * sizeof(unsigned long long)));
+  first_err(e, dalloc(s, (void **)&D.imp_st, (size_t)nd * sizeof(unsigned)));
   first_err(e, dalloc(s, (void **)&D.sync, SY_N * sizeof(unsigned)));
   first_err(e, dalloc(s, (void **)&D.fix_list, (size_t)nd * sizeof(int32_t)));
   if (ph->radviscosity || ph->dynamo) first_err(e, dalloc(s, (void **)&D.bl, (size_t)G.ncell * BL_NC * sizeof(double)));
@@ -1778,9 +1779,9 @@ static void launch_rijvisc(kz_sim *s, int dt_slot) {
 static ImpWork imp_work(const Dev &d, bool persist) {
   if (persist)
     return ImpWork{d.imp_uu00, d.imp_pp0, d.imp_aux, d.imp_slow, d.imp_list, d.imp_nslow, d.imp_ncnt, d.imp_rl,
-                   d.imp_rc, d.imp_qpos};
+                   d.imp_rc, d.imp_qpos, d.imp_st};
   return ImpWork{d.imp_uu00, d.imp_pp0, d.imp_aux, d.imp_slow, d.imp_list, d.imp_nslow, d.imp_ncnt, nullptr, nullptr,
-                 nullptr};
+                 nullptr, nullptr};
 }
 
 // persistent launches pay where the cells span many rounds of waves
@@ -2117,6 +2118,7 @@ int kz_group_set_runs(kz_group *G, kz_sim *const *sims, int nsims) {
     first_err(e, group_alloc(G, (void **)&G->w.rl, (size_t)2 * c * sizeof(int32_t)));
     first_err(e, group_alloc(G, (void **)&G->w.rc, 2 * sizeof(unsigned long long)));
     first_err(e, group_alloc(G, (void **)&G->w.qpos, 3 * sizeof(unsigned long long)));
+    first_err(e, group_alloc(G, (void **)&G->w.st, (size_t)c * sizeof(unsigned)));
     if (e) {
       group_free_work(G);
       return KZ_E_HIP;
@@ -2697,6 +2699,7 @@ kz_implicit_batch *kz_implicit_batch_create(int64_t n, const kz_physics *ph, int
   first_err(e, balloc(b, (void **)&b->w.rl, (size_t)2 * n * sizeof(int32_t)));
   first_err(e, balloc(b, (void **)&b->w.rc, 2 * sizeof(unsigned long long)));
   first_err(e, balloc(b, (void **)&b->w.qpos, 3 * sizeof(unsigned long long)));
+  first_err(e, balloc(b, (void **)&b->w.st, (size_t)n * sizeof(unsigned)));
   {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -2800,9 +2803,9 @@ int kz_implicit_batch_get(kz_implicit_batch *b, double *uu, double *pp, kz_impli
 // arrays, with every working buffer carved out of one static device array.
 // Per cell: the geometry planes (GEO_NC + 1), the SoA uu and pp (2 x 13),
 // the Newton reference state and start (2 x 13), the reference-state
-// scalars (IMP_NAUX) as doubles, and five int32 list entries.
+// scalars (IMP_NAUX) as doubles, and six int32 entries (lists, rung states).
 #define NA_DBL_PER_CELL (GEO_NC + 1 + 4 * NV + IMP_NAUX)
-#define NA_INT_PER_CELL 5
+#define NA_INT_PER_CELL 6
 #define NA_NCNT (NSLOT * SLOT_W + 8)  // cnt[NSLOT][SLOT_W] nslow ncnt rc[2] qpos[3], one spare
 static constexpr size_t NA_BYTES =
     ((size_t)KZ_NOALLOC_MAX_CELLS * (NA_DBL_PER_CELL * 8 + NA_INT_PER_CELL * 4) + NA_NCNT * 8 + 255) / 256 * 256;
@@ -2896,7 +2899,8 @@ extern "C" int kz_implicit_solve_noalloc(int64_t n, const double *pp_in, const k
   w.slow = ip;
   w.list = ip + n;
   w.rl = ip + 3 * n;
-  unsigned long long *ctr = (unsigned long long *)(((uintptr_t)(ip + 5 * n) + 7) & ~(uintptr_t)7);
+  w.st = (unsigned *)(ip + 5 * n);
+  unsigned long long *ctr = (unsigned long long *)(((uintptr_t)(ip + 6 * n) + 7) & ~(uintptr_t)7);
   unsigned long long *cnt = ctr;
   w.nslow = ctr + NSLOT * SLOT_W;
   w.ncnt = w.nslow + 1;
