@@ -153,6 +153,9 @@ KZDM double dm_log_entropy(double p, double rho, double indexn) {
     dm_log_dd(rho, &rh, &rl);
     return dm_log(dm_pow_from_log(ph, pl, indexn) / dm_pow_from_log(rh, rl, indexn + 1.0));
   }
+  // a negative pressure, as the trials of a damped W iteration meet it, has no
+  // power: NaN without the rest
+  if (p < 0.0 && kzm_isfinite(indexn) && __builtin_trunc(indexn) != indexn) return KZM_NAN;
   return kzm_log(kzm_pow(p, indexn) / kzm_pow(rho, indexn + 1.0));
 }
 
