@@ -949,22 +949,44 @@ __device__ __forceinline__ void bl_geo(const Dev &d, long n, long c, Geo &o) {
 // dynamo.zig:226-256 calcScaleHeight (single rank): per radial column the
 // density-weighted RMS of pi/2 - theta, summed in the reference's row order;
 // column 0 keeps the raw sum (the reference's gix > 0 condition).
-__global__ void __launch_bounds__(64) k_scale_height(GridD g, Dev d) {
-  const long ix = TID;
-  if (ix >= g.nx) return;
-  const long n = g.ncell;
+//
+// A block takes SH_COLS neighbouring columns and SH_ROWS rows of them at a
+// time: all threads form the terms of the tile (coalesced loads, many in
+// flight) in LDS, then one thread per column adds them in the serial order.
+// With one thread per column walking the rows, each of 384 threads waited for
+// its own loads row by row: 163 us per launch at 384x360 for 3.3 MB; 16
+// columns by 64 rows 24 us.
+constexpr int SH_COLS = 16, SH_ROWS = 64;
+__global__ void __launch_bounds__(256) k_scale_height(GridD g, Dev d) {
+  __shared__ double t0[SH_ROWS][SH_COLS + 1], t1[SH_ROWS][SH_COLS + 1];
+  const long n = g.ncell, rows = (long)g.ny * g.nz;
+  const int col = threadIdx.x % SH_COLS, r0 = threadIdx.x / SH_COLS;
+  const long ix = (long)blockIdx.x * SH_COLS + col;
   double sigma = 0, sth = 0;
-  for (long iy = 0; iy < g.ny; ++iy)
-    for (long iz = 0; iz < g.nz; ++iz) {
-      const long c = cidx(g, ix, iy, iz);
-      const double gd = d.gc[26 * n + c];
-      const double th = d.bl[BL_TH * n + c];
-      const double rho = d.p[RHO * n + c];
-      const double dth = KZ_PI / 2.0 - th;
-      sigma += rho * gd;
-      sth += rho * gd * dth * dth;
+  for (long base = 0; base < rows; base += SH_ROWS) {
+    for (int r = r0; r < SH_ROWS; r += 256 / SH_COLS) {
+      const long row = base + r;  // iy outermost, as the serial loop
+      if (ix < g.nx && row < rows) {
+        const long c = cidx(g, ix, row / g.nz, row % g.nz);
+        const double gd = d.gc[26 * n + c];
+        const double th = d.bl[BL_TH * n + c];
+        const double rho = d.p[RHO * n + c];
+        const double dth = KZ_PI / 2.0 - th;
+        t0[r][col] = rho * gd;
+        t1[r][col] = rho * gd * dth * dth;
+      }
     }
-  d.scaleth[ix] = ix > 0 ? kzm_sqrt(sth / sigma) : sth;
+    __syncthreads();
+    if (r0 == 0) {
+      const int m = rows - base < SH_ROWS ? (int)(rows - base) : SH_ROWS;
+      for (int r = 0; r < m; ++r) {
+        sigma += t0[r][col];
+        sth += t1[r][col];
+      }
+    }
+    __syncthreads();
+  }
+  if (r0 == 0 && ix < g.nx) d.scaleth[ix] = ix > 0 ? kzm_sqrt(sth / sigma) : sth;
 }
 // dynamo.zig:67-73 dampBphi
 __device__ __forceinline__ double damp_bphi(double alphabeta, double facradius, double faczh, double dt_over_pk,
@@ -1756,7 +1778,7 @@ static void launch_dynamo(kz_sim *s, int dt_slot, bool with_bc) {
   const GridD &g = s->g;
   {
     TimedLaunch tl(s, KZ_K_DYNAMO);
-    k_scale_height<<<nblk(g.nx, 64), 64, 0, s->stream>>>(g, s->d);
+    k_scale_height<<<nblk(g.nx, SH_COLS), 256, 0, s->stream>>>(g, s->d);
   }
   launch_set_bc(s);
   {
