@@ -114,6 +114,7 @@ __global__ void b_check_floors_rad(long n, double *pp, const kz_geom *g, kz_rad_
 __global__ void __launch_bounds__(64) b_implicit(long n, double *uu, double *pp, const kz_geom *g, const double *dt,
                                                  double gam, kz_rad_params rp, kz_opac_params op,
                                                  kz_implicit_params ip, kz_implicit_result *r) {
+  __shared__ NewtonLds lds;
   long i = TID;
   if (i >= n) return;
   Geo gm;
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(64) b_implicit(long n, double *uu, double *pp,
     p[k] = pp[i * NV + k];
     u[k] = uu[i * NV + k];
   }
-  r[i] = solve_implicit_lab(u, p, gm, dt[i], gam, rp, op, ip);
+  r[i] = solve_implicit_lab(lds, u, p, gm, dt[i], gam, rp, op, ip);
   for (int k = 0; k < NV; ++k) {
     pp[i * NV + k] = p[k];
     uu[i * NV + k] = u[k];

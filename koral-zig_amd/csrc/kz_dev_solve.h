@@ -637,8 +637,8 @@ struct ImpCtx {
 // implicit.zig:240-306 applyConstraints.  WP (the primitive block the
 // Newton solves for) is a template parameter so that every state index is
 // a compile-time constant and the 13-slot states stay in registers.
-template <int WP>
-KZD int apply_constraints(double *pp, double *uu, const double *uu0, const ImpCtx &cx) {
+template <int WP, class Uu0>
+KZDM int apply_constraints(double *pp, double *uu, const Uu0 &uu0, const ImpCtx &cx) {
   const Geo &gm = *cx.gm;
   double gdetu = gm.gdet, gi = 1.0 / gdetu;
   if (WP == WP_MHD) {
@@ -680,9 +680,9 @@ struct LagOpac {
 };
 
 // implicit.zig:337-427 residualG (scalar) on a filled state
-template <int WP, bool ALL>
-KZDM double residual(const double *uu, const double *pp, const RadState &st, const double *uu0, const State0 &s0,
-                    double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
+template <int WP, bool ALL, class Uu0>
+KZDM double residual(const double *uu, const double *pp, const RadState &st, const Uu0 &uu0, const State0 &s0,
+                     double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
   const Geo &gm = *cx.gm;
   double gdetu = gm.gdet;
   double dtau = dt / st.ucon[0];
@@ -734,8 +734,8 @@ KZDM double residual(const double *uu, const double *pp, const RadState &st, con
 // fills the state right after each applyConstraints and consumes it only
 // here, with pp unchanged in between, so filling at the point of use gives
 // the same values and keeps the state a temporary.
-template <int WP, bool ALL>
-KZDM double eval_residual_t(const double *uu, const double *pp, const LagOpac &lag, const double *uu0,
+template <int WP, bool ALL, class Uu0>
+KZDM double eval_residual_t(const double *uu, const double *pp, const LagOpac &lag, const Uu0 &uu0,
                             const State0 &s0, double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
   RadState st;
   fill_radstate_t<ALL>(pp, *cx.gm, cx.gam, *cx.op, we == WE_ENTROPY, st);
@@ -745,8 +745,8 @@ KZDM double eval_residual_t(const double *uu, const double *pp, const LagOpac &l
   }
   return residual<WP, ALL>(uu, pp, st, uu0, s0, dt, cx, we, wf, f);
 }
-template <int WP>
-KZDM double eval_residual(const double *uu, const double *pp, const LagOpac &lag, const double *uu0,
+template <int WP, class Uu0>
+KZDM double eval_residual(const double *uu, const double *pp, const LagOpac &lag, const Uu0 &uu0,
                           const State0 &s0, double dt, const ImpCtx &cx, int we, int wf, double f[4]) {
   return all_channels(*cx.op) ? eval_residual_t<WP, true>(uu, pp, lag, uu0, s0, dt, cx, we, wf, f)
                               : eval_residual_t<WP, false>(uu, pp, lag, uu0, s0, dt, cx, we, wf, f);
@@ -904,12 +904,27 @@ KZDM double fd_del(int j, double sign, const double *b, double eps, const Geo &g
 // lane (none now).  It also lets the lanes of a wave stand at different trial
 // states.  First rung at 384x360, with kz_dev_math.h: 262 -> 194 us.
 enum { AT_BASE = 0, AT_COL, AT_UPDATE };
+// What a Newton keeps for its whole length but reads once or twice per pass
+// lies in LDS, 40 doubles per lane (20 KB per wave, eight waves fill a CU's
+// 160 KB): the incoming conserved state, the reference-state scalars, the
+// residual at the base and the Jacobian.  With them in registers a lane
+// needed 350 to 450, one wave per SIMD, and the part past 256 was moved to
+// and fro between the two halves of the register file.
+enum { NL_JAC = 0, NL_F1 = 16, NL_UU0 = 20, NL_S0 = 33, NL_LAG = 36, NL_N = 40 };
+struct NewtonLds {
+  double v[NL_N][64];
+};
+// n values of the wave's LDS block as one lane's array
+struct LaneVec {
+  double *p;
+  __device__ __forceinline__ double operator[](int i) const { return p[i * 64]; }
+  __device__ __forceinline__ void put(int i, double x) const { p[i * 64] = x; }
+};
+KZDM LaneVec lane_vec(NewtonLds &l, int first) { return LaneVec{&l.v[first][threadIdx.x & 63]}; }
 struct NewtonState {
   double uu[NV], pp[NV];
   double b[4];        // the iteration's primitive block
   double rho0, en0;   // its density, and the energy density of the other block
-  double f1[4];       // residual at the base
-  double jac[4][4];   // Jacobian, then the scaled inverse that the update applies
   double errbase, del, xiapp;
   int iter, at, j;
   bool second;        // the column's second sign
@@ -923,26 +938,40 @@ KZDM void newton_start(NewtonState &n, const double *uu00, const double *pp0in) 
   n.iter = 0;
   n.at = AT_BASE;
 }
+// puts a cell's incoming state and reference scalars into its lane's LDS
+KZDM void newton_keep(NewtonLds &l, const double *uu00, const State0 &s0, const LagOpac &lag) {
+  const LaneVec u = lane_vec(l, NL_UU0), s = lane_vec(l, NL_S0), o = lane_vec(l, NL_LAG);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) u.put(i, uu00[i]);
+  s.put(0, s0.ehat);
+  s.put(1, s0.uint);
+  s.put(2, s0.sgas);
+  o.put(0, lag.kappaes);
+  o.put(1, lag.op.gas_abs);
+  o.put(2, lag.op.rad_abs);
+  o.put(3, lag.op.rad_ross);
+}
 // the update's trial state ppp - xiapp * (inverse) * f1
-KZDM void newton_update(NewtonState &n, double *blk) {
+KZDM void newton_update(NewtonState &n, NewtonLds &l, double *blk) {
+  const LaneVec jac = lane_vec(l, NL_JAC), f1 = lane_vec(l, NL_F1);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     double x = n.b[i];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x -= n.xiapp * n.jac[i][j] * n.f1[j];
+    for (int j = 0; j < 4; ++j) x -= n.xiapp * jac[i * 4 + j] * f1[j];
     blk[i] = x;
   }
 }
 template <int WP>
-KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, const State0 &s0, double dt,
-                    const ImpCtx &cx, int we, int wf) {
+KZDM int newton_pass(NewtonState &n, NewtonLds &l, double dt, const ImpCtx &cx, int we, int wf) {
   const kz_implicit_params &ip = *cx.ip;
   const Geo &gm = *cx.gm;
   double *uu = n.uu, *pp = n.pp;
   constexpr int sh = (WP == WP_MHD) ? UU : EE;
   constexpr int other = (WP == WP_MHD) ? EE : UU;
   double *blk = pp + sh;
-  const int fret = apply_constraints<WP>(pp, uu, uu00, cx);
+  const LaneVec uu0 = lane_vec(l, NL_UU0), jac = lane_vec(l, NL_JAC), f1 = lane_vec(l, NL_F1);
+  const int fret = apply_constraints<WP>(pp, uu, uu0, cx);
   if (n.at == AT_UPDATE) {
     bool ok = false;
     double edenmin = n.b[0] / ip.max_en_change_down;
@@ -962,7 +991,7 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
         n.xiapp /= ip.damping_factor;
       }
       if (n.xiapp < ip.max_damping) return -1;
-      newton_update(n, blk);
+      newton_update(n, l, blk);
       return 0;
     }
     double f3[4];
@@ -986,8 +1015,16 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
     set4(blk, n.j, get4(n.b, n.j) + n.del);
     return 0;
   }
-  double f[4];
-  const double err = eval_residual<WP>(uu, pp, lag, uu00, s0, dt, cx, we, wf, f);
+  double f[4], err;
+  {
+    asm volatile("" ::: "memory");  // read the LDS again rather than keep it through the constraints
+    const LaneVec s = lane_vec(l, NL_S0), o = lane_vec(l, NL_LAG);
+    const State0 s0{s[0], s[1], s[2]};
+    LagOpac lag;
+    lag.kappaes = o[0];
+    lag.op = Opac{o[1], o[2], o[3]};
+    err = eval_residual<WP>(uu, pp, lag, uu0, s0, dt, cx, we, wf, f);
+  }
   if (n.at == AT_BASE) {
     n.iter += 1;
     const double conv = (we == WE_ENTROPY) ? ip.entrconv : ip.conv;
@@ -996,7 +1033,7 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       n.b[i] = blk[i];
-      n.f1[i] = f[i];
+      f1.put(i, f[i]);
     }
     n.rho0 = pp[RHO];
     n.en0 = pp[other];
@@ -1004,7 +1041,7 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
     n.j = 0;
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) set4(n.jac[i], n.j, (f[i] - n.f1[i]) / n.del);
+    for (int i = 0; i < 4; ++i) jac.put(i * 4 + n.j, (f[i] - f1[i]) / n.del);
     set4(blk, n.j, get4(n.b, n.j));
     n.j += 1;
   }
@@ -1022,7 +1059,11 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
       isv[j] = 1.0 / sv[j];
     }
   }
-  double ij[4][4];
+  double ij[4][4], jm[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) jm[i][j] = jac[i * 4 + j];
   if (ip.jacobian_fp32) {
     // mixed precision: FP64 quotients rounded to FP32, scaled and
     // factored in FP32, the inverse applied in FP64
@@ -1030,7 +1071,7 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) jf[i][j] = (float)n.jac[i][j];
+      for (int j = 0; j < 4; ++j) jf[i][j] = (float)jm[i][j];
     if (ip.scale_jacobian) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -1049,28 +1090,29 @@ KZDM int newton_pass(NewtonState &n, const double *uu00, const LagOpac &lag, con
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (i != j) n.jac[i][j] = n.jac[i][j] * (sv[j] * isv[i]);
+          if (i != j) jm[i][j] = jm[i][j] * (sv[j] * isv[i]);
     }
-    invert4(n.jac, ij);
+    invert4(jm, ij);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) n.jac[i][j] = ip.scale_jacobian ? ij[i][j] * sv[i] * isv[j] : ij[i][j];
+    for (int j = 0; j < 4; ++j) jac.put(i * 4 + j, ip.scale_jacobian ? ij[i][j] * sv[i] * isv[j] : ij[i][j]);
   n.xiapp = 1.0;
   n.at = AT_UPDATE;
-  newton_update(n, blk);
+  newton_update(n, l, blk);
   return 0;
 }
 template <int WP>
-KZDM bool solve_4d_prim_core(const double *uu00, const LagOpac &lag, const State0 &s0,
-                                                          const double *pp0in, double dt, const ImpCtx &cx, int we,
-                                                          int wf, double *pp_out, int *iters_out) {
+KZDM bool solve_4d_prim_core(NewtonLds &l, const double *uu00, const LagOpac &lag, const State0 &s0,
+                             const double *pp0in, double dt, const ImpCtx &cx, int we, int wf, double *pp_out,
+                             int *iters_out) {
   NewtonState n;
+  newton_keep(l, uu00, s0, lag);
   newton_start(n, uu00, pp0in);
   int r;
   do {
-    r = newton_pass<WP>(n, uu00, lag, s0, dt, cx, we, wf);
+    r = newton_pass<WP>(n, l, dt, cx, we, wf);
   } while (r == 0);
   if (r < 0) return false;
 #pragma unroll
@@ -1080,7 +1122,7 @@ KZDM bool solve_4d_prim_core(const double *uu00, const LagOpac &lag, const State
 }
 
 // implicit.zig:927-1004 solveImplicitLab; returns kz_implicit_result
-KZD kz_implicit_result solve_implicit_lab(double *uu, double *pp, const Geo &gm, double dt, double gam,
+KZD kz_implicit_result solve_implicit_lab(NewtonLds &l, double *uu, double *pp, const Geo &gm, double dt, double gam,
                                           const kz_rad_params &rp, const kz_opac_params &op,
                                           const kz_implicit_params &ip) {
   kz_implicit_result fail = {0, -1, 0, WP_RAD, WE_ENERGY, WF_LAB};
@@ -1118,8 +1160,8 @@ KZD kz_implicit_result solve_implicit_lab(double *uu, double *pp, const Geo &gm,
       int wf = (ir == 0 || ir == 2) ? WF_LAB : WF_FF;
       double ppw[NV];
       int iters = 0;
-      bool ok = (wp == WP_MHD) ? solve_4d_prim_core<WP_MHD>(uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters)
-                               : solve_4d_prim_core<WP_RAD>(uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters);
+      bool ok = (wp == WP_MHD) ? solve_4d_prim_core<WP_MHD>(l, uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters)
+                               : solve_4d_prim_core<WP_RAD>(l, uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters);
       if (ok) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) pp[i] = ppw[i];

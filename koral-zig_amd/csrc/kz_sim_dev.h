@@ -179,6 +179,11 @@ static inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / b
 #ifndef KZ_WPE_RUNG0
 #define KZ_WPE_RUNG0 1
 #endif
+// Cells per lane of the chip at one wave per SIMD from which the first rung of
+// a grid is launched at two waves per SIMD (launch_implicit_br).
+#ifndef KZ_WIDE_ROUNDS
+#define KZ_WIDE_ROUNDS 3
+#endif
 #ifndef KZ_WPE_BC
 #define KZ_WPE_BC 1
 #endif

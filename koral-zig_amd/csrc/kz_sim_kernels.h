@@ -630,7 +630,7 @@ __device__ __forceinline__ void imp_load(const ImpWork &w, long nd, long t, doub
   lag.op.rad_ross = a[IA_KRR * nd + t];
 }
 template <class S, int WP>
-__device__ __forceinline__ void rung0_cell(const S &s, const ImpWork &w, const kz_physics &ph, long i) {
+__device__ __forceinline__ void rung0_cell(NewtonLds &l, const S &s, const ImpWork &w, const kz_physics &ph, long i) {
   constexpr int which = WP == WP_MHD ? 0 : 1;
   if (i >= (WP == WP_MHD ? n_mhd(w) : n_rad(w))) return;
   const long nd = s.count();
@@ -645,7 +645,7 @@ __device__ __forceinline__ void rung0_cell(const S &s, const ImpWork &w, const k
   ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
   int iters = 0;
   bool ok = ph.implicit.opdamp_maxlevels >= 0 &&
-            solve_4d_prim_core<WP>(uu00, lag, s0, pp0, dt, cx, WE_ENERGY, WF_LAB, ppw, &iters);
+            solve_4d_prim_core<WP>(l, uu00, lag, s0, pp0, dt, cx, WE_ENERGY, WF_LAB, ppw, &iters);
   if (ok) {
     s.solved(ph, t, gm, ppw, iters, 0, WP, WE_ENERGY, WF_LAB);
   } else {
@@ -655,13 +655,15 @@ __device__ __forceinline__ void rung0_cell(const S &s, const ImpWork &w, const k
 }
 // launched with nblk(n, 64) + 1 blocks: ceil(nrad/64) + ceil(nmhd/64) never
 // exceeds that for nrad + nmhd <= n
-template <class S, bool BR>
-__global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_rung0(S s, ImpWork w, kz_physics ph) {
+// W: waves per SIMD it is compiled for (launch_implicit_br).
+template <class S, bool BR, int W>
+__global__ void __launch_bounds__(64) KZ_WPE(W) k_imp_rung0(S s, ImpWork w, kz_physics ph) {
   ph.opac.synchrotron_bridge = BR;
+  __shared__ NewtonLds l;
   const long brad = (n_rad(w) + 63) / 64;
   const long b = blockIdx.x;
-  if (b < brad) rung0_cell<S, WP_RAD>(s, w, ph, b * 64 + threadIdx.x);
-  else rung0_cell<S, WP_MHD>(s, w, ph, (b - brad) * 64 + threadIdx.x);
+  if (b < brad) rung0_cell<S, WP_RAD>(l, s, w, ph, b * 64 + threadIdx.x);
+  else rung0_cell<S, WP_MHD>(l, s, w, ph, (b - brad) * 64 + threadIdx.x);
 }
 // Where a cell of the persistent first-rung launch goes when its Newton
 // ends: solved (recorded with the rung's attempt) or to the later rungs'
@@ -698,7 +700,7 @@ __device__ __forceinline__ int queue_lanes(long qlen) {
 // queue is exhausted; the loop ends when no lane holds a cell.  Every Newton
 // ends within maxiter + 1 steps and the queue is finite, so every wave exits.
 template <class S, int WP>
-__device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const kz_physics &ph, const int32_t *list,
+__device__ __forceinline__ void drain_queue(NewtonLds &l, const S &s, const ImpWork &w, const kz_physics &ph, const int32_t *list,
                                             long qlen, unsigned long long *qpos, int we, int wf,
                                             const RungDone<S> &done) {
   const int lane = threadIdx.x & 63;
@@ -708,9 +710,6 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
   long t = 0;
   double dt = 0;
   NewtonState ns;
-  double uu00[NV];
-  State0 s0;
-  LagOpac lag;
   Geo gm;
   for (;;) {
     const unsigned long long need = __ballot(!has && !exhausted);
@@ -726,8 +725,11 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
           done(list[q], gm, ns, false);  // the ladder has no level to run (implicit.zig:961)
         } else if (q < qlen) {
           t = list[q];
-          double pp0[NV];
+          double uu00[NV], pp0[NV];
+          State0 s0;
+          LagOpac lag;
           imp_load(w, nd, t, uu00, pp0, s0, lag);
+          newton_keep(l, uu00, s0, lag);
           s.geo(t, gm);
           dt = s.dt(t);
           const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
@@ -743,7 +745,7 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
     }
     if (has) {
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-      const int r = newton_pass<WP>(ns, uu00, lag, s0, dt, cx, we, wf);
+      const int r = newton_pass<WP>(ns, l, dt, cx, we, wf);
       if (r != 0) {
         done(t, gm, ns, r > 0);
         has = false;
@@ -755,11 +757,12 @@ __device__ __forceinline__ void drain_queue(const S &s, const ImpWork &w, const 
 template <class S, bool BR>
 __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_rung0_persist(S s, ImpWork w, kz_physics ph) {
   ph.opac.synchrotron_bridge = BR;
+  __shared__ NewtonLds l;
   const long nd = s.count();
   const RungDone<S> dr{&s, &w, &ph, 0, 1, WP_RAD, WE_ENERGY, WF_LAB};
-  drain_queue<S, WP_RAD>(s, w, ph, w.list + nd, n_rad(w), &w.qpos[0], WE_ENERGY, WF_LAB, dr);
+  drain_queue<S, WP_RAD>(l, s, w, ph, w.list + nd, n_rad(w), &w.qpos[0], WE_ENERGY, WF_LAB, dr);
   const RungDone<S> dm{&s, &w, &ph, 0, 0, WP_MHD, WE_ENERGY, WF_LAB};
-  drain_queue<S, WP_MHD>(s, w, ph, w.list, n_mhd(w), &w.qpos[1], WE_ENERGY, WF_LAB, dm);
+  drain_queue<S, WP_MHD>(l, s, w, ph, w.list, n_mhd(w), &w.qpos[1], WE_ENERGY, WF_LAB, dm);
 }
 // bits of ImpWork::st: RUNG_FAILED << r and RUNG_SOLVED << r for rung r = 1..5
 constexpr unsigned RUNG_FAILED = 1u, RUNG_SOLVED = 1u << 8, RUNG_FAILED_MASK = 0x3eu;
@@ -798,6 +801,7 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ULL << lane) - 1ULL;
   const long nd = s.count();
+  __shared__ NewtonLds l;
   const long n0 = (long)w.rc[0], m = n0 + (long)w.rc[1], qlen = 5 * m;
   // lanes for the two rungs that most of these cells need
   bool has = false, held = false, exhausted = qlen <= 0 || lane >= queue_lanes(2 * m);
@@ -805,9 +809,6 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
   int ir = 1, wp = WP_MHD, we = WE_ENERGY, wf = WF_FF;
   double dt = 0;
   NewtonState ns;
-  double uu00[NV];
-  State0 s0;
-  LagOpac lag;
   Geo gm;
   for (;;) {
     const unsigned long long need = __ballot(!has && !exhausted);
@@ -830,8 +831,11 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
               w.slow[k] = (int32_t)t;
             }
           } else if (!rung_solved_below(w, t, ir)) {
-            double pp0[NV];
+            double uu00[NV], pp0[NV];
+            State0 s0;
+            LagOpac lag;
             imp_load(w, nd, t, uu00, pp0, s0, lag);
+            newton_keep(l, uu00, s0, lag);
             s.geo(t, gm);
             dt = s.dt(t);
             wp = (ir == 1 || ir == 4) ? sw : ot;
@@ -850,8 +854,9 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
     }
     if (has && !held) {
       const ImpCtx cx{&gm, ph.gam, &ph.rad, &ph.opac, &ph.implicit, 1.0};
-      const int r = (wp == WP_MHD) ? newton_pass<WP_MHD>(ns, uu00, lag, s0, dt, cx, we, wf)
-                                   : newton_pass<WP_RAD>(ns, uu00, lag, s0, dt, cx, we, wf);
+      int r = 0;
+      if (wp == WP_MHD) r = newton_pass<WP_MHD>(ns, l, dt, cx, we, wf);
+      if (wp == WP_RAD) r = newton_pass<WP_RAD>(ns, l, dt, cx, we, wf);
       if (r > 0) {
         atomicOr(&w.st[t], RUNG_SOLVED << ir);
         held = true;
@@ -883,6 +888,7 @@ __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(
 template <class S, bool BR>
 __global__ void __launch_bounds__(64) k_imp_slow(S s, ImpWork w, kz_physics ph, int first_level) {
   ph.opac.synchrotron_bridge = BR;
+  __shared__ NewtonLds l;
   long i = TID;
   // the first-rung lists have been consumed; clear them for the next pass
   if (i == 0) *w.ncnt = 0;
@@ -910,8 +916,8 @@ __global__ void __launch_bounds__(64) k_imp_slow(S s, ImpWork w, kz_physics ph, 
       int wf = (ir == 0 || ir == 2) ? WF_LAB : WF_FF;
       double ppw[NV];
       int iters = 0;
-      bool ok = (wp == WP_MHD) ? solve_4d_prim_core<WP_MHD>(uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters)
-                               : solve_4d_prim_core<WP_RAD>(uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters);
+      bool ok = (wp == WP_MHD) ? solve_4d_prim_core<WP_MHD>(l, uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters)
+                               : solve_4d_prim_core<WP_RAD>(l, uu00, lag, s0, pp0, dt, cx, we, wf, ppw, &iters);
       if (ok) {
         s.solved(ph, t, gm, ppw, iters, ir, wp, we, wf);
         return;
@@ -937,7 +943,14 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
     k_imp_ladder_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 1);
   } else {
-    k_imp_rung0<S, BR><<<nb + 1, 64, 0, st>>>(cells, w, ph);
+    // Two waves per SIMD hide each other's latencies at the price of 95 spilled
+    // registers: where the cells fill the chip several times over that wins,
+    // with fewer the chain of the longest solve sets the time and a wave is
+    // better off alone.  Whole implicit pass, one and two waves: 256x256 166
+    // and 179 us, 384x360 288 and 299, 512x400 391 and 383, 128x128x16 531 and
+    // 476, 128x128x32 938 and 858.
+    if (n >= KZ_WIDE_ROUNDS * 64L * persist_blocks) k_imp_rung0<S, BR, 2><<<nb + 1, 64, 0, st>>>(cells, w, ph);
+    else k_imp_rung0<S, BR, KZ_WPE_RUNG0><<<nb + 1, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 0);
   }
 }

@@ -1806,12 +1806,10 @@ static ImpWork imp_work(const Dev &d, bool persist) {
                  nullptr, nullptr};
 }
 
-// persistent launches pay where the cells span many rounds of waves
-// (192x192x64: 11.4 -> 10.6 ms of implicit work per step); at 384x360
-// (two rounds) the merged launch is faster (0.85 against 0.91 ms)
-static bool imp_persistent(long n, unsigned persist_blocks, int imp_launch) {
-  return imp_launch == 2 || (imp_launch == 0 && n >= 8L * 64 * (long)persist_blocks);
-}
+// Grids and groups run the persistent launches only when asked to: their cells
+// need one to four iterations, and the merged first rung takes less at every
+// size (128x128x32: 656 us per pass against 800, 384x360 194 against 300).
+static bool imp_persistent(int imp_launch) { return imp_launch == 2; }
 // The implicit kernels over the n cells of a cell source (a grid, or the
 // runs of a group); the bridge variants are in kz_options.hip.
 extern "C++" template <class S>
@@ -1828,7 +1826,7 @@ static void launch_op_implicit(kz_sim *s, int dt_slot) {
   if (!s->ph.has_opac) return;
   {
     TimedLaunch tl(s, KZ_K_IMPLICIT);
-    const bool persist = imp_persistent(ndom(s), s->persist_blocks, s->imp_launch);
+    const bool persist = imp_persistent(s->imp_launch);
     launch_implicit(GridCells{s->g, s->d, dt_slot}, imp_work(s->d, persist), s->ph, ndom(s), persist,
                     s->persist_blocks, s->stream);
   }
@@ -2192,7 +2190,7 @@ static int group_fork(kz_group *G) {
 }
 static void group_implicit(kz_group *G, int dt_slot) {
   if (!G->ph.has_opac || G->n == 0) return;
-  const bool persist = imp_persistent(G->n, G->persist_blocks, G->imp_launch);
+  const bool persist = imp_persistent(G->imp_launch);
   launch_implicit(MultiCells{G->runs, (int)G->sims.size(), G->n, dt_slot}, G->w, G->ph, G->n, persist,
                   G->persist_blocks, G->stream);
 }
