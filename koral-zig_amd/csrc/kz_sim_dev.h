@@ -100,6 +100,18 @@ __device__ __forceinline__ long fidx(const GridD &g, int d, long ix, long iy, lo
   long jx = ix + g.ngx, jy = iy + g.ngy, jz = iz + g.ngz;
   return (jz * g.fsy[d] + jy) * (long)g.fsx[d] + jx;
 }
+// t = i0 + n0 * (i1 + n1 * i2).  Counts of cells, faces and corners fit 32 bits
+// with room to spare (a cell takes over 3 KB of device memory), and a 64-bit
+// division is some 100 instructions, of which a kernel's index took three to
+// eight (k_face_flux 13 394 -> 11 489 instructions, 57.0 -> 54.9 us per launch
+// at 384x360).  GridCells keeps the 64-bit form: with this one the first rung
+// at two waves per SIMD spilled more, 656 -> 716 us at 128x128x32.
+__device__ __forceinline__ void split3(long t, long n0, long n1, long &i0, long &i1, long &i2) {
+  const unsigned u = (unsigned)t, q = u / (unsigned)n0, z = q / (unsigned)n1;
+  i0 = u - q * (unsigned)n0;
+  i1 = q - z * (unsigned)n1;
+  i2 = z;
+}
 __device__ __forceinline__ double xl_(const GridD &g, long i) { return g.minx + (double)i * g.dx; }
 __device__ __forceinline__ double yl_(const GridD &g, long i) { return g.miny + (double)i * g.dy; }
 __device__ __forceinline__ double zl_(const GridD &g, long i) { return g.minz + (double)i * g.dz; }

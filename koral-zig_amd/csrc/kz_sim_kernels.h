@@ -21,7 +21,11 @@ __device__ __forceinline__ void wavespeeds_pass(const GridD &g, const Dev &d, co
   long lx = act[0], ly = act[1], lz = act[2];
   long wx = g.nx + 2 * lx, wy = g.ny + 2 * ly, wz = g.nz + 2 * lz;
   if (t >= wx * wy * wz) return;
-  long ix = t % wx - lx, iy = (t / wx) % wy - ly, iz = t / (wx * wy) - lz;
+  long ix, iy, iz;
+  split3(t, wx, wy, ix, iy, iz);
+  ix -= lx;
+  iy -= ly;
+  iz -= lz;
   long n = g.ncell;
   long c = cidx(g, ix, iy, iz);
   double pp[NV];
@@ -97,7 +101,8 @@ __device__ __forceinline__ void u2p_pass(const GridD &g, const Dev &d, const kz_
   long nd = (long)g.nx * g.ny * g.nz;
   const bool fix_hd = ph.do_fixups, fix_rad = ph.do_fixups && ph.do_u2prad_fixups;
   if (t < nd) {
-    long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+    long ix, iy, iz;
+    split3(t, g.nx, g.ny, ix, iy, iz);
     long c = cidx(g, ix, iy, iz);
     long n = g.ncell;
     double uu[NV], pp[NV];
@@ -197,7 +202,7 @@ template <int DIM>
 struct FaceTile {
   static constexpr int c0d = DIM == 0 ? 1 : 0, c1d = DIM == 2 ? 1 : 2;
   long wf, w0, l0, l1;
-  long t0, r0, e0;  // x runs: first face, its row, its left cell's place in rows of wf + 1 cells
+  long t0, r0, p0;  // x runs: first face, its row and its place in the row
   long x0, i0, c1;  // y/z tiles: first column, first face along DIM, the other cross index
   int nface, ncell;
   __device__ FaceTile(const GridD &g, const FaceTiles &ft, long b) {
@@ -211,27 +216,27 @@ struct FaceTile {
       t0 = b * ft.fx;
       const long left = wf * w0 * w1 - t0;
       nface = (int)(left < ft.fx ? left : ft.fx);
-      r0 = t0 / wf;
-      e0 = r0 * (wf + 1) + t0 % wf;
+      r0 = (unsigned)t0 / (unsigned)wf;
+      p0 = t0 - r0 * wf;
       ncell = right(nface - 1) + 1;
     } else {
       const long ntx = (w0 + FT_T - 1) / FT_T, nti = (wf + FT_F - 1) / FT_F;
-      x0 = (b % ntx) * FT_T;
-      i0 = ((b / ntx) % nti) * FT_F;
-      c1 = b / (ntx * nti) + l1;
+      split3(b, ntx, nti, x0, i0, c1);
+      x0 *= FT_T;
+      i0 *= FT_F;
+      c1 += l1;
       nface = FT_T * FT_F;
       ncell = FT_T * (FT_F + 1);
     }
   }
-  __device__ int left(int f) const { return DIM == 0 ? (int)(f + (t0 + f) / wf - r0) : f; }
+  __device__ int left(int f) const { return DIM == 0 ? f + (int)((unsigned)(p0 + f) / (unsigned)wf) : f; }
   __device__ int right(int f) const { return DIM == 0 ? left(f) + 1 : f + FT_T; }
   __device__ bool face(int f, long cell[3]) const {
     if (f >= nface) return false;
     if (DIM == 0) {
-      const long t = t0 + f;
-      cell[0] = t % wf;
-      cell[1] = (t / wf) % w0 + l0;
-      cell[2] = t / (wf * w0) + l1;
+      split3(t0 + f, wf, w0, cell[0], cell[1], cell[2]);
+      cell[1] += l0;
+      cell[2] += l1;
       return true;
     }
     const long x = x0 + f % FT_T, i = i0 + f / FT_T;
@@ -244,10 +249,10 @@ struct FaceTile {
   __device__ bool cellk(int k, long cell[3]) const {
     if (k >= ncell) return false;
     if (DIM == 0) {
-      const long e = e0 + k, r = e / (wf + 1);
-      cell[0] = e % (wf + 1) - 1;
-      cell[1] = r % w0 + l0;
-      cell[2] = r / w0 + l1;
+      split3(r0 * (wf + 1) + p0 + k, wf + 1, w0, cell[0], cell[1], cell[2]);
+      cell[0] -= 1;
+      cell[1] += l0;
+      cell[2] += l1;
       return true;
     }
     const long x = x0 + k % FT_T, i = i0 - 1 + k / FT_T;

@@ -25,7 +25,8 @@
 __global__ void k_p2u_domain(GridD g, Dev d, double gam) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   long c = cidx(g, ix, iy, iz);
   Geo gm;
   geo_c(g, d, ix, iy, iz, gm);
@@ -415,7 +416,8 @@ __device__ bool fixup_slots(const GridD &g, const Dev &d, const kz_physics &ph, 
   return true;
 }
 __device__ void fixup_cell(const GridD &g, const Dev &d, const kz_physics &ph, long t, bool hd, bool rad) {
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   if (polar_row(ph, g, iy)) return;
   long n = g.ncell;
   long c = cidx(g, ix, iy, iz);
@@ -451,7 +453,8 @@ __global__ void __launch_bounds__(256) k_u2p_fixups(GridD g, Dev d, kz_physics p
 __global__ void __launch_bounds__(256) k_fixup(GridD g, Dev d, kz_physics ph, int which) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   long n = g.ncell;
   long c = cidx(g, ix, iy, iz);
   if (d.flags[which * n + c] == 0) return;
@@ -486,7 +489,8 @@ __device__ __forceinline__ double gdet_pb(const GridD &g, const Dev &d, int iv, 
 __global__ void __launch_bounds__(256) k_divb(GridD g, Dev d, double *out) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   double divb;
   if (g.nz == 1) {
     divb = (gdet_pb(g, d, B1, ix, iy, iz) + gdet_pb(g, d, B1, ix, iy - 1, iz) - gdet_pb(g, d, B1, ix - 1, iy, iz) -
@@ -527,7 +531,8 @@ __global__ void k_emf(GridD g, Dev d) {
   long t = TID;
   long nx = g.nx, ny = g.ny, nz = g.nz;
   if (t >= (nx + 1) * (ny + 1) * (nz + 1)) return;
-  long ix = t % (nx + 1), iy = (t / (nx + 1)) % (ny + 1), iz = t / ((nx + 1) * (ny + 1));
+  long ix, iy, iz;
+  split3(t, nx + 1, ny + 1, ix, iy, iz);
   double c1 = (ny > 1 && nz > 1) ? 0.25 : 0.5, c2 = (nx > 1 && nz > 1) ? 0.25 : 0.5,
          c3 = (nx > 1 && ny > 1) ? 0.25 : 0.5;
   long e = eidx(g, ix, iy, iz);
@@ -583,7 +588,7 @@ __global__ void __launch_bounds__(128) KZ_WPE(KZ_WPE_UPDATE) k_update(GridD g, D
   const long n = g.ncell;
   const double dt = d.ss[sslot];
   if (live) {
-    ix = t % g.nx; iy = (t / g.nx) % g.ny; iz = t / ((long)g.nx * g.ny);
+    split3(t, g.nx, g.ny, ix, iy, iz);
     c = cidx(g, ix, iy, iz);
   }
   if (live && side == 0) {
@@ -888,7 +893,11 @@ __global__ void __launch_bounds__(64) k_rijvisc(GridD g, Dev d, kz_physics ph, i
   const long lx = g.nx > 1, ly = g.ny > 1, lz = g.nz > 1;
   const long wx = g.nx + 2 * lx, wy = g.ny + 2 * ly, wz = g.nz + 2 * lz;
   if (t >= wx * wy * wz) return;
-  const long ix = t % wx - lx, iy = (t / wx) % wy - ly, iz = t / (wx * wy) - lz;
+  long ix, iy, iz;
+  split3(t, wx, wy, ix, iy, iz);
+  ix -= lx;
+  iy -= ly;
+  iz -= lz;
   if (is_corner(g, ix, iy, iz)) return;
   const long n = g.ncell, c = cidx(g, ix, iy, iz);
   const double global_dt = d.ss[sslot];
@@ -1036,7 +1045,11 @@ __global__ void __launch_bounds__(64) k_dynamo_a(GridD g, Dev d, kz_physics ph, 
   const long lx = g.nx > 1, ly = g.ny > 1, lz = g.nz > 1;
   const long wx = g.nx + 2 * lx, wy = g.ny + 2 * ly, wz = g.nz + 2 * lz;
   if (t >= wx * wy * wz) return;
-  const long ix = t % wx - lx, iy = (t / wx) % wy - ly, iz = t / (wx * wy) - lz;
+  long ix, iy, iz;
+  split3(t, wx, wy, ix, iy, iz);
+  ix -= lx;
+  iy -= ly;
+  iz -= lz;
   const long n = g.ncell, c = cidx(g, ix, iy, iz);
   const double dt = d.ss[sslot];
   Geo geom, gbl;
@@ -1100,7 +1113,8 @@ __device__ __forceinline__ double corner_a(const GridD &g, const Dev &d, long ix
 __global__ void __launch_bounds__(128) k_dynamo_curl(GridD g, Dev d, kz_physics ph) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  const long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   const long n = g.ncell, c = cidx(g, ix, iy, iz);
   const bool d3 = g.nz > 1;
   // the A_r and A_theta corners are averages of zeros
@@ -1157,7 +1171,8 @@ __global__ void __launch_bounds__(128) k_dynamo_curl(GridD g, Dev d, kz_physics 
 // cells, so only domain cells are copied.
 __device__ __forceinline__ bool dom_cell(const GridD &g, long t, long &c) {
   if (t >= (long)g.nx * g.ny * g.nz) return false;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   c = cidx(g, ix, iy, iz);
   return true;
 }
@@ -1252,7 +1267,8 @@ __global__ void k_end_step(GridD g, Dev d, kz_physics ph) {
   long t = TID;
   if (t == 0) d.ss[SS_T] = d.ss[SS_T] + d.ss[SS_DT];
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   long n = g.ncell;
   long c = cidx(g, ix, iy, iz);
   double pp[NV], uu[NV];
@@ -1271,7 +1287,8 @@ __global__ void k_end_step(GridD g, Dev d, kz_physics ph) {
 __global__ void k_beta_max(GridD g, Dev d, kz_physics ph, unsigned long long *out) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   long c = cidx(g, ix, iy, iz);
   double pp[NV];
   ld(d.p, g.ncell, c, pp);
@@ -1290,7 +1307,8 @@ __global__ void k_beta_max(GridD g, Dev d, kz_physics ph, unsigned long long *ou
 __global__ void k_beta_scale(GridD g, Dev d, kz_physics ph, double fac) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   long n = g.ncell;
   long c = cidx(g, ix, iy, iz);
   double pp[NV], uu[NV];
@@ -1308,7 +1326,8 @@ __global__ void k_beta_scale(GridD g, Dev d, kz_physics ph, double fac) {
 __global__ void k_init_tsd(GridD g, Dev d, double tsd) {
   long t = TID;
   if (t >= (long)g.nx * g.ny * g.nz) return;
-  long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   d.scal[SC_TSTEPDEN * g.ncell + cidx(g, ix, iy, iz)] = tsd;
   if (t == 0) {
     for (int k = 0; k < NSLOT; ++k)
@@ -2372,7 +2391,8 @@ __global__ void __launch_bounds__(128) k_scalar_terms(GridD g, Dev d, kz_physics
   long t = TID;
   const long nd = (long)g.nx * g.ny * g.nz;
   if (t >= nd) return;
-  const long ix = t % g.nx, iy = (t / g.nx) % g.ny, iz = t / ((long)g.nx * g.ny);
+  long ix, iy, iz;
+  split3(t, g.nx, g.ny, ix, iy, iz);
   const long n = g.ncell, c = cidx(g, ix, iy, iz);
   const long ns = (long)g.nz * g.ny, sh = iz * g.ny + iy;
   const bool twod = g.nz == 1;
