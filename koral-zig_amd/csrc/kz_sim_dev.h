@@ -170,8 +170,8 @@ static inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / b
 // Minimum waves per SIMD each heavy kernel is compiled for (1 = no bound;
 // n bounds the kernel to 512/n vector registers).  Chosen by a measured
 // sweep at 384x360: 2 waves help the memory-bound update and u2p passes and
-// the implicit preparation (their register need is just above 256); the face
-// flux and the first Newton rung lose more to spills than they gain.
+// the implicit preparation; the first Newton rung gains from two waves only
+// on large grids (KZ_WIDE_ROUNDS).
 #define KZ_WPE(n) __attribute__((amdgpu_waves_per_eu(n)))
 #ifndef KZ_WPE_FACE
 #define KZ_WPE_FACE 2

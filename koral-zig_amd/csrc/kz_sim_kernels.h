@@ -389,11 +389,11 @@ __global__ void __launch_bounds__(128) KZ_WPE(KZ_WPE_FACE) k_face_flux(GridD g, 
 //   k_imp_slow     rungs 1..5 (and damped-opacity levels) for the cells the
 //                  first rung did not solve, gathered into a list
 // Batches, whose cells need from one to forty iterations per rung, run the
-// first rung and then each later rung of level 0 as persistent work-stealing
-// launches (k_imp_rung0_persist, k_imp_rung_persist): every lane holds one
-// cell's Newton state and takes the next cell of the queue when its cell is
-// solved or has failed, so a wave's time is its lanes' total iterations, not
-// 64 times its slowest cell's; k_imp_slow then takes the damped levels.
+// first rung and then the later rungs of level 0 as persistent work-stealing
+// launches (k_imp_rung0_persist, k_imp_ladder_persist): every lane holds one
+// cell's Newton state and takes the next entry of the queue when its Newton
+// ends, so a wave's time is its lanes' total iterations, not 64 times its
+// slowest cell's; k_imp_slow then takes the damped levels.
 // The sequence of attempts per cell is the reference ladder's; inputs to
 // every rung are the stored reference-state values, so results equal the
 // single-pass ladder bit for bit.

@@ -265,7 +265,7 @@ class Sim:
         _chk(lib().kz_sim_replay(self.h), "kz_sim_replay")
 
     def set_implicit_launch(self, mode):
-        """0 by size, 1 merged first-rung launch, 2 persistent work stealing."""
+        """0 (default) and 1 merged first-rung launch, 2 persistent work stealing."""
         _chk(lib().kz_sim_set_implicit_launch(self.h, int(mode)), "kz_sim_set_implicit_launch")
 
     def busy(self):

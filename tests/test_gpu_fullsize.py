@@ -4,8 +4,8 @@
   perturbation 0x4b5a4d493335355f): two CFL steps, state, flags and clock
   bit for bit, the implicit pass in the launch shape chosen by size.
 * 192x192x64 wedge (a = 0.9375, periodic phi, rho and u perturbed): one
-  CFL step bit for bit, the implicit pass in the persistent launch shape
-  its size selects.
+  CFL step bit for bit, the implicit pass in the launch its size selects
+  (the first rung at two waves per SIMD).
 * calcDivB (koral/sim/ct.zig:336-381) on the device equals the oracle's bit
   for bit, and after twenty GPU steps the corner divergence stays at machine
   precision: everywhere in 2D, and in 3D away from the periodic phi seam and

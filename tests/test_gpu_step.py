@@ -162,7 +162,7 @@ def test_set_time_resume():
 @pytest.mark.parametrize("mode", [1, 2])
 def test_implicit_launch_shapes(mode):
     """Both launch shapes of the implicit pass (one merged first-rung launch;
-    persistent work stealing, which large grids use) give the oracle's steps
+    persistent work stealing, as batches use it) give the oracle's steps
     bit for bit, with radiative viscosity and the dynamo on."""
     grid = T.grid_puffy(40, 36)
     phys = T.physics_puffy(radviscosity=True, dynamo=True)
