@@ -6,6 +6,7 @@
 Both are compiled with -ffp-contract=off: no fused multiply-adds anywhere,
 so device and host arithmetic round exactly as written.
 """
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -14,6 +15,9 @@ import tempfile
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
+_spec = importlib.util.spec_from_file_location("kz_asmcheck", HERE / "asmcheck.py")  # with or without the package
+asmcheck = importlib.util.module_from_spec(_spec)
+_spec.loader.exec_module(asmcheck)
 ROOT = HERE.parent
 LIB = HERE / "lib"
 HIP_SOURCES = [HERE / "csrc" / "kz_step.hip", HERE / "csrc" / "kz_options.hip", HERE / "csrc" / "kz_cellops.hip"]
@@ -28,7 +32,9 @@ HIPCC_FLAGS = [
     "-Wno-unused-result",
     # constants stay where they are used: hoisted out of the solver loops they
     # need more registers than there are, and each is then read back from a
-    # spill (k_u2p: 256 vector registers and 140 B of scratch against 247)
+    # spill (k_u2p: 256 vector registers and 140 B of scratch against 247).
+    # Without the flag the synchrotron-bridge ladder kernels spill vectors
+    # ahead of an exec restore and give wrong results: asmcheck refuses them
     "-mllvm", "-disable-machine-licm",
 ]
 
@@ -48,9 +54,10 @@ def _run(cmd):
 
 
 def compile_hip(out, defines=None):
-    """Compile every HIP source to an object of its own, in parallel, and
-    link them into the shared library `out`.  `defines` maps macro names to
-    values (the tuner's knobs)."""
+    """Compile every HIP source to an object of its own, in parallel, search
+    the assembly that each came from (asmcheck), and link the objects into the
+    shared library `out`.  `defines` maps macro names to values (the tuner's
+    knobs)."""
     out = Path(out)
     dflags = [f"-D{k}={v}" for k, v in (defines or {}).items()]
     cflags = [f for f in HIPCC_FLAGS if f != "-shared"]
@@ -59,7 +66,7 @@ def compile_hip(out, defines=None):
         for src in HIP_SOURCES:
             obj = Path(td) / (src.stem + ".o")
             objs.append(obj)
-            cmd = [_hipcc(), *cflags, *dflags, "-c", "-o", str(obj), str(src)]
+            cmd = [_hipcc(), *cflags, *dflags, "-save-temps=obj", "-c", "-o", str(obj), str(src)]
             procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         failed = []
         for cmd, p in procs:
@@ -69,6 +76,13 @@ def compile_hip(out, defines=None):
                 failed.append(" ".join(map(str, cmd)))
         if failed:
             raise RuntimeError("build failed: " + "; ".join(failed))
+        lost = []
+        for obj in objs:
+            asm = obj.with_name(f"{obj.stem}-hip-amdgcn-amd-amdhsa-{ARCH}.s")
+            lost += [f"{fn} {block}: {'; '.join(ins[:4])}" for fn, block, ins in asmcheck.lost_lanes(asm.read_text())]
+        if lost:
+            raise RuntimeError("the compiler spills vectors ahead of an exec restore, so the build would give wrong "
+                               "results in:\n  " + "\n  ".join(lost))
         tmp = out.with_name(out.name + ".tmp")
         _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])
         os.replace(tmp, out)
