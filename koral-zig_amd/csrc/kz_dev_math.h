@@ -25,6 +25,17 @@ namespace kzd {
 
 KZDM double dm_sel(bool c, double a, double b) { return c ? a : b; }
 
+// x toward zero as an integer for every x: past the range the nearest value in
+// it, 0 for NaN, which is what the instruction gives.  A cast is undefined for
+// those operands (dm_exp_dd selects its result only afterwards), and what keeps
+// them from one costs: taking the low word of x + 1.5 * 2^52 made 40
+// steps at 128x128x32 2.3 % and a batch of 2^19 cells 4 % slower.
+KZDM int dm_int(double x) {
+  int k;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(k) : "v"(x));
+  return k;
+}
+
 // kzm_exp_dd
 KZDM double dm_exp_dd(double x, double xl) {
   const double t = x * KZM_INV_LN2;
@@ -47,7 +58,7 @@ KZDM double dm_exp_dd(double x, double xl) {
   q = KZM_FMA(r, q, 0.5);
   q = (r * r) * q;
   const double y = 1.0 + (r + (q + c * (1.0 + r)));
-  const double v = __builtin_amdgcn_ldexp(y, (int)kd);
+  const double v = __builtin_amdgcn_ldexp(y, dm_int(kd));
   return dm_sel(x > 709.782712893384, KZM_INF, dm_sel(x < -745.1332191019412, 0.0, v));
 }
 KZDM double dm_exp(double x) { return dm_exp_dd(x, 0.0); }

@@ -66,3 +66,12 @@ def test_radstate_corners(channels):
             c, z = c[:, :8], z[:, :8]
         bad = np.nonzero(~((c == z) | (np.isnan(c) & np.isnan(z))).all(axis=1))[0]
         assert bad.size == 0, (full, rows[bad[0]], c[bad[0]], z[bad[0]])
+
+
+def test_exp_outside_the_integers():
+    """Operands whose quotient by ln 2 no integer holds: NaN, infinities and
+    everything past 1.5e9."""
+    x = np.array([np.nan, np.inf, -np.inf, 1e9, -1e9, 1.5e9, -1.5e9, 2e9, -2e9, 1e19, -1e19, 1e300, -1e300,
+                  np.finfo(float).max, -np.finfo(float).max])
+    c, g = kzo.math_fn("exp", x), hip.math_fn("exp", x)
+    assert np.array_equal(c, g, equal_nan=True), (c, g)
