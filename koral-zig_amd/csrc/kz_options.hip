@@ -35,8 +35,8 @@ void opt_launch_face_flux(const GridD &g, const Dev &d, const kz_physics &ph, co
 
 template <class S>
 void opt_launch_implicit_bridge(const S &cells, const ImpWork &w, const kz_physics &ph, long n, bool persist,
-                                unsigned persist_blocks, hipStream_t st) {
-  launch_implicit_br<S, true>(cells, w, ph, n, persist, persist_blocks, st);
+                                unsigned ncu, hipStream_t st) {
+  launch_implicit_br<S, true>(cells, w, ph, n, persist, ncu, st);
 }
 template void opt_launch_implicit_bridge<GridCells>(const GridCells &, const ImpWork &, const kz_physics &, long, bool,
                                                     unsigned, hipStream_t);

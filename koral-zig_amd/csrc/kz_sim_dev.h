@@ -171,7 +171,7 @@ static inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / b
 // n bounds the kernel to 512/n vector registers).  Chosen by a measured
 // sweep at 384x360: 2 waves help the memory-bound update and u2p passes and
 // the implicit preparation; the first Newton rung gains from two waves only
-// on large grids (KZ_WIDE_ROUNDS).
+// on large grids (wide_cells).
 #define KZ_WPE(n) __attribute__((amdgpu_waves_per_eu(n)))
 #ifndef KZ_WPE_FACE
 #define KZ_WPE_FACE 2
@@ -191,11 +191,6 @@ static inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / b
 #ifndef KZ_WPE_RUNG0
 #define KZ_WPE_RUNG0 1
 #endif
-// Cells per lane of the chip at one wave per SIMD from which the first rung of
-// a grid is launched at two waves per SIMD (launch_implicit_br).
-#ifndef KZ_WIDE_ROUNDS
-#define KZ_WIDE_ROUNDS 3
-#endif
 #ifndef KZ_WPE_BC
 #define KZ_WPE_BC 1
 #endif
@@ -205,5 +200,11 @@ static inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / b
 #ifndef KZ_PERSIST_PER_CU
 #define KZ_PERSIST_PER_CU 4
 #endif
+// Cells from which the first rung of a grid or a group is launched at two
+// waves per SIMD: three for every lane of a chip of ncu CUs that holds one wave
+// per SIMD (launch_implicit_br).  It counts the SIMDs, not the blocks of a
+// batch's persistent launches, whose width is tuned by itself.
+constexpr long SIMD_PER_CU = 4, WIDE_ROUNDS = 3;
+constexpr long wide_cells(long ncu) { return WIDE_ROUNDS * 64 * SIMD_PER_CU * ncu; }
 
 #endif

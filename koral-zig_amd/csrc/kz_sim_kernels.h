@@ -939,11 +939,11 @@ __global__ void __launch_bounds__(64) k_imp_slow(S s, ImpWork w, kz_physics ph, 
 // `persist`.
 template <class S, bool BR>
 static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physics &ph, long n, bool persist,
-                               unsigned persist_blocks, hipStream_t st) {
+                               unsigned ncu, hipStream_t st) {
   const unsigned nb = nblk(n, 64);
   k_imp_prep<S, BR><<<nb, 64, 0, st>>>(cells, w, ph);
   if (persist) {
-    const unsigned np = persist_blocks < (unsigned long)n ? persist_blocks : (unsigned)n;
+    const unsigned width = KZ_PERSIST_PER_CU * ncu, np = width < (unsigned long)n ? width : (unsigned)n;
     k_imp_rung0_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_ladder_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 1);
@@ -954,7 +954,7 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
     // better off alone.  Whole implicit pass, one and two waves: 256x256 166
     // and 179 us, 384x360 288 and 299, 512x400 391 and 383, 128x128x16 531 and
     // 476, 128x128x32 938 and 858.
-    if (n >= KZ_WIDE_ROUNDS * 64L * persist_blocks) k_imp_rung0<S, BR, 2><<<nb + 1, 64, 0, st>>>(cells, w, ph);
+    if (n >= wide_cells(ncu)) k_imp_rung0<S, BR, 2><<<nb + 1, 64, 0, st>>>(cells, w, ph);
     else k_imp_rung0<S, BR, KZ_WPE_RUNG0><<<nb + 1, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 0);
   }
@@ -966,6 +966,6 @@ void opt_launch_face_flux(const GridD &g, const Dev &d, const kz_physics &ph, co
                           hipStream_t st);
 template <class S>
 void opt_launch_implicit_bridge(const S &cells, const ImpWork &w, const kz_physics &ph, long n, bool persist,
-                                unsigned persist_blocks, hipStream_t st);
+                                unsigned ncu, hipStream_t st);
 
 #endif

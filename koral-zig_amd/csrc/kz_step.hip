@@ -1382,8 +1382,8 @@ struct kz_sim {
   size_t dev_bytes = 0;
   double *scal_buf = nullptr;  // per-cell terms of the scalar diagnostics (allocated on first use)
   double wedge = 0;            // maxz - minz of the caller's grid
-  unsigned persist_blocks = 1024;  // one wave per SIMD for the persistent implicit launches
-  int imp_launch = 0;              // 0 by size, 1 merged first rung, 2 persistent
+  unsigned ncu = 256;  // CUs of the device: the implicit launches' shape
+  int imp_launch = 0;  // kz_sim_set_implicit_launch: 0 and 1 merged first rung, 2 persistent
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   int graph_steps = 0;
@@ -1510,7 +1510,7 @@ kz_sim *kz_sim_create(const kz_grid *gr, const kz_physics *ph, const double *g, 
   {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
-      s->persist_blocks = (unsigned)(KZ_PERSIST_PER_CU * ncu);
+      s->ncu = (unsigned)ncu;
   }
   GridD &G = s->g;
   G.nx = gr->nx; G.ny = gr->ny; G.nz = gr->nz; G.ng = gr->ng;
@@ -1833,9 +1833,9 @@ static bool imp_persistent(int imp_launch) { return imp_launch == 2; }
 // runs of a group); the bridge variants are in kz_options.hip.
 extern "C++" template <class S>
 static void launch_implicit(const S &cells, const ImpWork &w, const kz_physics &ph, long n, bool persist,
-                            unsigned persist_blocks, hipStream_t st) {
-  if (ph.opac.synchrotron_bridge) opt_launch_implicit_bridge(cells, w, ph, n, persist, persist_blocks, st);
-  else launch_implicit_br<S, false>(cells, w, ph, n, persist, persist_blocks, st);
+                            unsigned ncu, hipStream_t st) {
+  if (ph.opac.synchrotron_bridge) opt_launch_implicit_bridge(cells, w, ph, n, persist, ncu, st);
+  else launch_implicit_br<S, false>(cells, w, ph, n, persist, ncu, st);
 }
 static void launch_radimp_fixup(kz_sim *s) {
   if (s->ph.has_opac && s->ph.do_fixups && s->ph.do_radimp_fixups)
@@ -1847,7 +1847,7 @@ static void launch_op_implicit(kz_sim *s, int dt_slot) {
     TimedLaunch tl(s, KZ_K_IMPLICIT);
     const bool persist = imp_persistent(s->imp_launch);
     launch_implicit(GridCells{s->g, s->d, dt_slot}, imp_work(s->d, persist), s->ph, ndom(s), persist,
-                    s->persist_blocks, s->stream);
+                    s->ncu, s->stream);
   }
   launch_radimp_fixup(s);
 }
@@ -2061,7 +2061,7 @@ struct kz_group {
   long n = 0, cap_n = 0;
   ImpWork w{};
   std::vector<void *> wallocs;
-  unsigned persist_blocks = 1024;
+  unsigned ncu = 256;
   int imp_launch = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
@@ -2108,7 +2108,7 @@ int kz_group_create(kz_group **out) {
     kz_group_destroy(G);
     return KZ_E_HIP;
   }
-  G->persist_blocks = (unsigned)(ncu > 0 ? KZ_PERSIST_PER_CU * ncu : 1024);
+  if (ncu > 0) G->ncu = (unsigned)ncu;
   *out = G;
   return 0;
 }
@@ -2211,7 +2211,7 @@ static void group_implicit(kz_group *G, int dt_slot) {
   if (!G->ph.has_opac || G->n == 0) return;
   const bool persist = imp_persistent(G->imp_launch);
   launch_implicit(MultiCells{G->runs, (int)G->sims.size(), G->n, dt_slot}, G->w, G->ph, G->n, persist,
-                  G->persist_blocks, G->stream);
+                  G->ncu, G->stream);
 }
 // nsteps CFL steps of every run: the kernel sequence of launch_step per run,
 // with both implicit passes of each step taken by the group's launches
@@ -2687,7 +2687,7 @@ struct kz_implicit_batch {
   std::vector<void *> allocs;
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool has_input = false;
-  unsigned persist_blocks = 1024;
+  unsigned ncu = 256;
 };
 
 static int balloc(kz_implicit_batch *b, void **p, size_t bytes) {
@@ -2744,7 +2744,7 @@ kz_implicit_batch *kz_implicit_batch_create(int64_t n, const kz_physics *ph, int
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       first_err(e, KZ_E_HIP);
-    b->persist_blocks = (unsigned)(ncu > 0 ? KZ_PERSIST_PER_CU * ncu : 1024);  // one wave per SIMD
+    if (ncu > 0) b->ncu = (unsigned)ncu;
   }
   for (auto &x : b->ev) first_err(e, hip_err(hipEventCreate(&x)));
   if (e) {
@@ -2798,7 +2798,7 @@ int kz_implicit_batch_solve(kz_implicit_batch *b, double *ms) {
   k_batch_reset<<<nblk(n < NSLOT * SLOT_W ? NSLOT * SLOT_W : n, 256), 256, 0, b->stream>>>(n, b->pp_in, b->pp, b->uu, b->res, b->cnt);
   const BatchCells cells{n, b->gp, b->dt, b->uu, b->pp, b->res, b->cnt};
   HIPCHK(hipEventRecord(b->ev[0], b->stream));
-  launch_implicit(cells, b->w, b->ph, n, true, b->persist_blocks, b->stream);
+  launch_implicit(cells, b->w, b->ph, n, true, b->ncu, b->stream);
   HIPCHK(hipEventRecord(b->ev[1], b->stream));
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(b->stream));
@@ -2895,7 +2895,7 @@ __global__ void k_na_unpack(long n, const double *uu, const double *pp, double *
 namespace {
 struct NaDevice {
   unsigned char *base = nullptr;  // this device's copy of `scratch`
-  unsigned blocks = 0;            // persistent launch width: one wave per SIMD
+  unsigned ncu = 0;               // CUs: the persistent launches' width
 };
 std::mutex na_mu;
 NaDevice na_dev[64];
@@ -2922,7 +2922,7 @@ extern "C" int kz_implicit_solve_noalloc(int64_t n, const double *pp_in, const k
       if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr) return KZ_E_HIP;
       int ncu = 0;
       if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return KZ_E_HIP;
-      na_dev[dev].blocks = (unsigned)(ncu > 0 ? KZ_PERSIST_PER_CU * ncu : 1024);
+      na_dev[dev].ncu = (unsigned)(ncu > 0 ? ncu : 256);
       na_dev[dev].base = (unsigned char *)ptr;
     }
     nd = na_dev[dev];
@@ -2949,7 +2949,7 @@ extern "C" int kz_implicit_solve_noalloc(int64_t n, const double *pp_in, const k
   kz_physics ph = *phys;
   k_na_pack<<<nblk(n < NA_NCNT ? NA_NCNT : n, 256), 256, 0, st>>>(n, pp_in, g, gp, spp, suu, res, ctr);
   const BatchCells cells{n, gp, dt, suu, spp, res, cnt};
-  launch_implicit(cells, w, ph, n, true, nd.blocks, st);
+  launch_implicit(cells, w, ph, n, true, nd.ncu, st);
   k_na_unpack<<<nblk(n * NV, 256), 256, 0, st>>>(n, suu, spp, uu, pp, cnt, counts);
   return hipGetLastError() == hipSuccess ? KZ_OK : KZ_E_HIP;
 }
