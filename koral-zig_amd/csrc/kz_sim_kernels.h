@@ -418,6 +418,7 @@ struct ImpWork {
 // are skipped, dt is a step scalar, a solved cell stores u and p and clears
 // its radimp flag (sim.zig:1762-1768), a failed one sets it to -1.
 struct GridCells {
+  static constexpr bool PERSIST_ONLY = false;
   GridD g;
   Dev d;
   int sslot;
@@ -463,6 +464,7 @@ struct GridCells {
 // n independent cells (solveImplicitLab per record, implicit.zig:927-1009):
 // geometry planes and dt per cell, the ladder's outcome recorded per cell.
 struct BatchCells {
+  static constexpr bool PERSIST_ONLY = true;
   long n;
   const double *gp;   // [GEO_NC + 1][n]: the geometry planes, then x1
   const double *dtv;  // [n]
@@ -499,6 +501,7 @@ struct RunCells {
   long off;
 };
 struct MultiCells {
+  static constexpr bool PERSIST_ONLY = false;
   const RunCells *r;  // [nr], off ascending, r[0].off == 0
   int nr;
   long n;
@@ -942,12 +945,13 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
                                unsigned ncu, hipStream_t st) {
   const unsigned nb = nblk(n, 64);
   k_imp_prep<S, BR><<<nb, 64, 0, st>>>(cells, w, ph);
-  if (persist) {
+  // batches know no other shape: their merged kernels would be reached by nothing
+  if (persist || S::PERSIST_ONLY) {
     const unsigned width = KZ_PERSIST_PER_CU * ncu, np = width < (unsigned long)n ? width : (unsigned)n;
     k_imp_rung0_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_ladder_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 1);
-  } else {
+  } else if constexpr (!S::PERSIST_ONLY) {
     // Two waves per SIMD hide each other's latencies at the price of 95 spilled
     // registers: where the cells fill the chip several times over that wins,
     // with fewer the chain of the longest solve sets the time and a wave is
