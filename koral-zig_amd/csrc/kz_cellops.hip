@@ -231,6 +231,17 @@ __global__ void b_radstate(long n, const double *pp, const kz_geom *g, double ga
   o[9] = calc_chi_slim(pp + i * NV, gm, gam, op);
 }
 
+// a^b by the functions that the opacities and the entropy call: their
+// branch-free powers where those are defined (a positive exponent that is no
+// integer; a negative one of a positive finite base), else kz_math.h's
+__device__ double math_pow(double a, double b) {
+  if (!kzm_isfinite(b) || kzm_is_int(b)) return kzm_pow(a, b);
+  if (b > 0.0) return dm_pow_frac(a, b);
+  if (!(a > 0.0 && a < KZM_INF)) return kzm_pow(a, b);
+  double h, l;
+  dm_log_dd(a, &h, &l);
+  return dm_pow_from_log(h, l, b);
+}
 __global__ void b_math(long n, int fn, const double *x, const double *y, double *out) {
   long i = TID;
   if (i >= n) return;
@@ -238,7 +249,7 @@ __global__ void b_math(long n, int fn, const double *x, const double *y, double 
   switch (fn) {
     case 0: r = dm_exp(a); break;
     case 1: r = dm_log(a); break;
-    case 2: r = kzm_pow(a, b); break;
+    case 2: r = math_pow(a, b); break;
     case 3: r = dm_cbrt(a); break;
     case 4: r = dm_log1p(a); break;
     case 5: r = kzm_sqrt(a); break;

@@ -75,3 +75,33 @@ def test_exp_outside_the_integers():
                   np.finfo(float).max, -np.finfo(float).max])
     c, g = kzo.math_fn("exp", x), hip.math_fn("exp", x)
     assert np.array_equal(c, g, equal_nan=True), (c, g)
+
+
+@pytest.mark.parametrize("y", [0.2, 0.86, 4.0 / 3.0, 1.0 / 3.0, 0.69, 1.69, 0.463, -0.463, 1.5, 2.5, -7.5, 40.5])
+def test_pow_edges(y):
+    """The exponents of the opacities and of the entropy, and two whose results
+    over- and underflow: subnormal, zero, negative, infinite and NaN bases."""
+    x = np.concatenate([EDGES["log"], EDGES["cbrt"], [1.0, -1.0, 0.0, -0.0, np.inf, -np.inf, np.nan, 1.7976931348623157e308],
+                        10.0 ** np.linspace(-323.0, 308.0, 4001)])
+    c, g = kzo.math_fn("pow", x, y), hip.math_fn("pow", x, y)
+    bad = np.nonzero(~((c.view(np.int64) == g.view(np.int64)) | (np.isnan(c) & np.isnan(g))))[0]
+    assert bad.size == 0, (y, x[bad[:5]], c[bad[:5]], g[bad[:5]])
+
+
+@pytest.mark.parametrize("gam", [5.0 / 3.0, 4.0 / 3.0, 1.5, 2.0, 1.2])
+def test_entropy_edges(gam):
+    """The entropy of a state over densities and internal energies from
+    subnormal to huge, zero, negative, infinite and NaN; 1.5 and 2 make its
+    exponent 1 / (gam - 1) an integer, which takes the general power."""
+    v = np.concatenate([[0.0, -0.0, 5e-324, 2.0 ** -1022, 1.0, -1e-10, -1e30, np.inf, -np.inf, np.nan,
+                         1.7976931348623157e308], 10.0 ** np.arange(-320.0, 308.0, 23.0),
+                        10.0 ** np.linspace(-30.0, 30.0, 25)])
+    inp, _ = read_kgld("rad/rad_thermo.kgld", 36, 13)
+    pp = np.repeat(inp[:1, 23:36], v.size ** 2, axis=0)
+    pp[:, 0], pp[:, 1] = np.repeat(v, v.size), np.tile(v, v.size)
+    geo = np.repeat(geoms(inp[:1]), len(pp), axis=0)
+    op = T.opac_params_puffy()
+    c, g = kzo.radstate(pp, geo, gam, op, 1)[:, 13], hip.radstate(pp, geo, gam, op, 1)[:, 8]
+    bad = np.nonzero(~((c == g) | (np.isnan(c) & np.isnan(g))))[0]
+    assert bad.size == 0, (gam, pp[bad[0], :2], c[bad[0]], g[bad[0]])
+    assert np.isfinite(c).sum() > 100
