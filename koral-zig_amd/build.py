@@ -32,7 +32,9 @@ HIPCC_FLAGS = [
     "-Wno-unused-result",
     # constants stay where they are used: hoisted out of the solver loops they
     # need more registers than there are, and each is then read back from a
-    # spill (k_u2p: 256 vector registers and 140 B of scratch against 247).
+    # spill (k_u2p: 256 vector registers and 140 B of scratch against 249, 30.1
+    # against 25.5 us at 384x360; the two-wave first rung 754 against 636 us at
+    # 128x128x32; the one-wave one 1 to 2 % the other way).
     # Without the flag the synchrotron-bridge ladder kernels spill vectors
     # ahead of an exec restore and give wrong results: asmcheck refuses them
     "-mllvm", "-disable-machine-licm",

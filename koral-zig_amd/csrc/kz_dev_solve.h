@@ -899,7 +899,7 @@ KZDM double fd_del(int j, double sign, const double *b, double eps, const Geo &g
 //
 // One pass per trial state, so that the constraints and the residual stand in
 // the code once each.  Written out per use (three and two copies per
-// primitive block) the first rung's code was 293 KB (145 KB now) against the
+// primitive block) the first rung's code was 293 KB (142 KB now) against the
 // 64 KB of instruction cache that two CUs share, with 400 B of scratch per
 // lane (none now).  It also lets the lanes of a wave stand at different trial
 // states.  First rung at 384x360, with kz_dev_math.h: 262 -> 194 us.

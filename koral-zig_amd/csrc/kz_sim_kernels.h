@@ -800,8 +800,9 @@ __device__ __forceinline__ bool rung_solved_below(const ImpWork &w, long t, int 
 //
 // Bound by the serial chain of the longest ladder: run one after the other by
 // one lane per cell, the five rungs of the slowest cell set the time of every
-// batch.  Per solve, with queue_lanes: 59 -> 9 ms at 4099 cells (480 of them
-// here), 148 -> 49 ms at 2^19.  In the independent-cell batch rung 1 fails for 93 % of these cells and rung 2 then
+// batch.  This launch, with queue_lanes: 69 -> 8 ms at 4099 cells (480 of them
+// here), 148 -> 40 ms at 2^19; the first rung is another 8 and 36 ms.  In the
+// independent-cell batch rung 1 fails for 93 % of these cells and rung 2 then
 // solves 96 %, so little is tried in vain.
 template <class S, bool BR>
 __global__ void __launch_bounds__(64) KZ_WPE(KZ_WPE_RUNG0) k_imp_ladder_persist(S s, ImpWork w, kz_physics ph) {
@@ -952,10 +953,11 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
     k_imp_ladder_persist<S, BR><<<np, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 1);
   } else if constexpr (!S::PERSIST_ONLY) {
-    // Two waves per SIMD hide each other's latencies at the price of 95 spilled
-    // registers: where the cells fill the chip several times over that wins,
-    // with fewer the chain of the longest solve sets the time and a wave is
-    // better off alone.  Whole implicit pass, one and two waves: 256x256 166
+    // Two waves per SIMD hide each other's latencies at the price of 167 spilled
+    // vector registers (384 B of scratch per lane; 157 to 189 over the cell
+    // sources and the bridge): where the cells fill the chip several times over
+    // that wins, with fewer the chain of the longest solve sets the time and a
+    // wave is better off alone.  Whole implicit pass, one and two waves: 256x256 166
     // and 179 us, 384x360 288 and 299, 512x400 391 and 383, 128x128x16 531 and
     // 476, 128x128x32 938 and 858.
     if (n >= wide_cells(ncu)) k_imp_rung0<S, BR, 2><<<nb + 1, 64, 0, st>>>(cells, w, ph);
