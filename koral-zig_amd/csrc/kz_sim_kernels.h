@@ -957,9 +957,13 @@ static void launch_implicit_br(const S &cells, const ImpWork &w, const kz_physic
     // vector registers (384 B of scratch per lane; 157 to 189 over the cell
     // sources and the bridge): where the cells fill the chip several times over
     // that wins, with fewer the chain of the longest solve sets the time and a
-    // wave is better off alone.  Whole implicit pass, one and two waves: 256x256 166
-    // and 179 us, 384x360 288 and 299, 512x400 391 and 383, 128x128x16 531 and
-    // 476, 128x128x32 938 and 858.
+    // wave is better off alone.  Whole implicit pass, one and two
+    // waves: 256x256 166 and 179 us, 384x360 288 and 299, 512x384 383 and 364,
+    // 512x400 422 and 382, 128x128x16 528 and 463, 128x128x32 932 and 820.  With
+    // the bridge 512x384 413 and 417, 512x400 461 and 450, 128x128x16 567 and
+    // 535, 128x128x32 1005 and 960.  A step of a run group, without and with the
+    // bridge: three 256x256 runs 1645 and 1646 us, 1735 and 1737; two 384x360
+    // runs 1930 and 1892, 2026 and 1988.
     if (n >= wide_cells(ncu)) k_imp_rung0<S, BR, 2><<<nb + 1, 64, 0, st>>>(cells, w, ph);
     else k_imp_rung0<S, BR, KZ_WPE_RUNG0><<<nb + 1, 64, 0, st>>>(cells, w, ph);
     k_imp_slow<S, BR><<<nb, 64, 0, st>>>(cells, w, ph, 0);
